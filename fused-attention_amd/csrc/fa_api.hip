@@ -120,6 +120,36 @@ int fwd_block_m(int block_m, int /*block_n*/, int /*D*/, int gh) {
   if (gh == 4) return 64;  // four heads run 64-row tiles (fwd_heads_per_wg)
   return (block_m == 64 && gh == 1) ? 128 : block_m;
 }
+// Forward instance of a call.  Below a grid that fills the GPU the keys of a tile are split
+// over groups of waves (fwd_kernel's KS): the call then waits for the serial chain of the
+// last rows, and every other CU, or SIMD of a CU, idles.  By the number W of 64-row
+// workgroups, which depends on neither tile_m nor H_kv (results still depend on neither):
+//   W <= one per CU:  D <= 64: 32 rows x 4 groups over 128-key tiles; D = 128, whose 128-key
+//     tiles allow one workgroup per CU: 64 rows x 4 groups
+//   W <= three per CU, S >= 512 (below, a chain is a few tiles and the merge costs as much:
+//     B=16 H=32 S=64 D=64 5.2 -> 5.4 us, B=16 H=8 S=384 D=128 15.3 -> 15.5): 64 rows x 2 groups
+//     over 64-key tiles (D = 128 at S >= 4096 and W <= two per CU: 64 x 4 again)
+// Measured, us of unsplit / 64 x 2 / 64 x 4 / 32 x 4 (x: not an instance):
+//   D = 64:  B=2 H=8 S=512 (W = 128) 8.6 / 6.6 / 6.9 / 5.8; B=8 H=1 S=1755 (224) 18.7 / 13.4 / 11.8 /
+//   10.8; B=1 H=2 S=8192 (256) 68.8 / 48.3 / 36.9 / 34.5; B=2 H=8 S=2048 (512) 21.5 / 16.2 / 17.8 / 19.0;
+//   B=2 H=16 S=1024 (512) 13.2 / 9.9 / 13.4 / 13.3
+//   D = 128: B=3 H=5 S=1000 (240) 17.6 / 15.0 / 15.1 / 17.8; B=1 H=1 S=16384 (256) 201 / 153 / 120 / 119;
+//   B=2 H=8 S=2048 (512) 31.2 / 28.1 / 28.0 / 43.7; B=1 H=8 S=4096 (512) 56.2 / 49.7 / 44.3 / 68.0;
+//   GQA B=1 H=32 H_kv=8 S=1531 (768) 30.1 / 27.9 / 36.0 / 55.6; B=2 H=16 S=2048 (1024) 41.9 / 44.1 / 54 / 88
+//   and through this rule, us before / after: D = 32: B=2 H=8 S=512 7.3 / 5.4, S=1024 10.8 / 6.0, B=1 H=4
+//   S=4096 31.2 / 13.9, B=2 H=8 S=2048 18.0 / 12.4; B=3 H=8 S=2048 (768): D = 32 25.2 / 16.1, D = 64
+//   32.6 / 21.9, D = 128 46.7 / 34.9; B=3 H=16 S=1024 (768): D = 64 19.7 / 16.1, D = 128 27.8 / 23.5
+struct FwdShape {
+  int block_m, block_n, gh;   // gh = -KS: key groups
+};
+bool fwd_key_split(int B, int H, int S, int D, FwdShape* out) {
+  const long long w = (long long)B * H * ((S + 63) / 64), cus = cu_count();
+  if (w > 3 * cus || (w > cus && S < 512)) return false;
+  const bool four = w <= cus || (D == 128 && S >= 4096 && w <= 2 * cus);
+  if (out) *out = !four ? FwdShape{64, 64, -2} : D == 128 ? FwdShape{64, 128, -4} : FwdShape{32, 128, -4};
+  return true;
+}
+
 int dq_block_m(int block_m, int /*D*/) { return block_m == 64 ? 128 : block_m; }
 
 // Work items (key-tile chunks) the dK/dV kernel should have for its heavy-first order
@@ -222,8 +252,12 @@ int fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   if (st != FA_OK) return st;
   if (H_kv <= 0 || H_kv > H || H % H_kv != 0) return FA_ERR_DIMS;
   if (!q || !k || !v || !o) return FA_ERR_NULL;
-  const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, block_n);
-  fa::FwdFn fn = fwd_table(dtype, D, fwd_block_m(block_m, block_n, D, gh), block_n, gh, lse != nullptr);
+  FwdShape w;
+  if (!fwd_key_split(B, H, S, D, &w)) {
+    const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, block_n);
+    w = FwdShape{fwd_block_m(block_m, block_n, D, gh), block_n, gh};
+  }
+  fa::FwdFn fn = fwd_table(dtype, D, w.block_m, w.block_n, w.gh, lse != nullptr);
   if (!fn) return FA_ERR_UNSUPPORTED;
   fa::FwdArgs a{q, k, v, o, lse, B, H, H_kv, S, D, scale_log2, hip_stream};
   return fn(a);
@@ -315,6 +349,8 @@ int fa_fwd_exact(const void* q, const void* k, const void* v, void* o, float* ls
   if (!q || !k || !v || !o) return FA_ERR_NULL;
   fa::FwdFn fn = fwd_table(dtype, D, block_m, block_n, heads_per_wg, lse != nullptr);
   if (!fn) return FA_ERR_UNSUPPORTED;
+  FwdShape w;
+  if (fwd_key_split(B, H, S, D, &w)) fn = fwd_table(dtype, D, w.block_m, w.block_n, w.gh, lse != nullptr);
   fa::FwdArgs a{q, k, v, o, lse, B, H, H_kv, S, D, scale_log2, hip_stream};
   return fn(a);
 }

@@ -41,6 +41,11 @@
 //     the mask applied arithmetically, and a wave whose rows lie wholly before the
 //     last tile skips it.  The first reference point is S(0)'s row max, so no
 //     tile starts on the rescale path.
+//   * grids that leave the GPU idle (few heads, short sequences) split the keys of every
+//     tile over KS groups of waves: group k computes its share of each tile's keys against
+//     a reference point and sums of its own, and the groups' (m, l, acc) are merged through
+//     LDS at the end.  A row block's serial chain of key tiles, which is what such a grid
+//     waits for, is then KS times shorter per tile or KS times as many waves share it.
 //   * heavy-first, XCD-aware order: the 8 XCDs each take a contiguous range of
 //     (batch, head-group) units and dispatch the heaviest (last) query tiles of
 //     all their units first.
@@ -73,9 +78,9 @@ constexpr int kWaitVmcnt0 = 0x0F70;
 #endif
 constexpr float kSumLimit = float(1 << FA_RESCALE_THRESHOLD);
 
-template <int D, int BM, int BN, int GH>
+template <int D, int BM, int BN, int GH, int KS>
 constexpr int fwd_waves_per_simd() {
-  return (BN == 64 && (BM / 32) * GH >= 4) ? 2 : 1;
+  return (BN / KS <= 64 && (BM / 32) * GH * KS >= 4) ? 2 : 1;
 }
 
 // Compile-time marker of a pipeline iteration that runs wholly below the diagonal.
@@ -92,15 +97,16 @@ __device__ __forceinline__ u32x4 lds_read_tr16x2(const unsigned char* base, int 
   return u32x4{ua[0], ua[1], ub[0], ub[1]};
 }
 
-template <typename E, int D, int BM, int BN, int GH, bool LSE>
-__global__ __launch_bounds__(64 * (BM / 32) * GH)
-__attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd<D, BM, BN, GH>(), fwd_waves_per_simd<D, BM, BN, GH>())))
+// KS > 1: the keys of every tile are split over KS groups of WR waves (GH = 1).
+template <typename E, int D, int BM, int BN, int GH, int KS, bool LSE>
+__global__ __launch_bounds__(64 * (BM / 32) * GH * KS)
+__attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd<D, BM, BN, GH, KS>(), fwd_waves_per_simd<D, BM, BN, GH, KS>())))
 void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
                 const uint16_t* __restrict__ V, uint16_t* __restrict__ O, float* __restrict__ Lse,
-                int B, int H, int Hkv, int S, float scale_log2) {
+                int B, int H, int Hkv, int S, float scale_log2, int first) {
   constexpr int WR = BM / 32;
-  constexpr int NW = WR * GH;
-  constexpr int NB = BN / 32;          // 32-key blocks per tile
+  constexpr int NW = WR * GH * KS;
+  constexpr int NB = BN / 32 / KS;     // 32-key blocks of a tile per wave
   constexpr int KT = D / 16;           // MFMA k-steps over D
   constexpr int DB = D / 32;           // 32-row blocks of O^T
   constexpr int ROWB = D * 2;          // bytes per K/V row
@@ -109,6 +115,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   constexpr int CPR = ROWB / 16;       // 16-byte chunks per row
   constexpr int NDMA = (NBLK + NW - 1) / NW;  // DMA blocks per wave per tile (K and V each)
   static_assert(TILE % 1024 == 0, "tile must be whole 1 KB DMA blocks");
+  static_assert(KS == 1 || GH == 1, "key groups serve one head");
   const float NEG_INF = -__builtin_inff();
 
   // K buffers at [0, 2 TILE), V buffers at [2 TILE, 4 TILE)
@@ -118,7 +125,9 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, hh = lane >> 5;
-  const int wh = wave % GH, wr = wave / GH;
+  const int wh = wave % GH, wr = wave / GH % WR;
+  const int kg = KS > 1 ? wave / WR : 0;   // this wave's key group
+  const int kw = kg * (32 * NB);           // and its first key in a tile
 
   // ---- work item: (batch, head group, query tile).  Workgroups reach the 8 XCDs
   // round-robin (wg % 8); XCD x takes a contiguous range of units (its own L2 keeps
@@ -132,7 +141,14 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   const int nunits = B * units_per_b;
   const int wg = blockIdx.x;
   int unit, qt;
-  if (nunits % 8 == 0) {
+  if constexpr (KS > 1) {
+    // heaviest first over all heads (with a multiple of 8 heads an XCD still serves its own);
+    // when every workgroup is resident at once, the second one of a CU (from `first` on) in
+    // reverse, the lightest beside the heaviest (+1 to +4 % at B=2 H=8 S=2048, B=1 H=8 S=4096)
+    const int L = first > 0 && wg >= first ? first + (int)gridDim.x - 1 - wg : wg;
+    unit = L % nunits;
+    qt = nq - 1 - L / nunits;
+  } else if (nunits % 8 == 0) {
     const int per = nunits / 8, i = wg / 8;
     const int G = xcd_group(per, nq);
     const int grp = i / (G * nq), r = i % (G * nq);
@@ -206,7 +222,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   // K A-operand, k-step t: row c (+ 32 nb), chunk (2t+hh) ^ kswz(c)
   int koff[KT];
 #pragma unroll
-  for (int t = 0; t < KT; ++t) koff[t] = c * ROWB + (((2 * t + hh) ^ ((c * CPR / 16) & (CPR - 1))) << 4);
+  for (int t = 0; t < KT; ++t) koff[t] = (kw + c) * ROWB + (((2 * t + hh) ^ ((c * CPR / 16) & (CPR - 1))) << 4);
   // V^T A-operand via transposed reads: in 16-lane group G, lane (kr, c4) addresses
   // key row 4hh + kr (+ block offsets) and the 4 columns feeding output lanes
   // 4c4..4c4+3, which hold d = pi(16(G&1) + 4c4) + 0..3 of the 32-d block.
@@ -215,7 +231,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     const int G = lane >> 4, kr = (lane >> 2) & 3, c4 = lane & 3;
     const int e = 2 * pi_swap23(16 * (G & 1) + 4 * c4);     // byte offset < 64
     const int k1 = (ROWB >= 128) ? (kr >> 1) : 0;
-    const int base = (4 * hh + kr) * ROWB + (e ^ (32 * (kr & 1)));
+    const int base = (kw + 4 * hh + kr) * ROWB + (e ^ (32 * (kr & 1)));
     voff_even = base + 64 * k1;           // (64 db + e) ^ 32 kr for even db, minus 64 db
     voff_odd = base + 64 * (1 - k1) - 64;  // same for odd db
   }
@@ -261,7 +277,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   auto mask_tile = [&](f32x16 (&s)[NB], int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      const int t = q0 - k0 - 32 * nb;
+      const int t = q0 - k0 - kw - 32 * nb;
 #pragma unroll
       for (int g = 0; g < 16; ++g)
         if (lane_kq > t - (8 * (g >> 2) + (g & 3))) s[nb][g] = NEG_INF;
@@ -399,6 +415,9 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   s_tile(Kbuf(0), sa);
   if (jfull == 0) mask_tile(sa, 0);
   mrun = tile_max(sa);
+  // (a key group that meets no key of its rows in tile 0 has no finite score: a finite
+  // reference point keeps its P at zero, and a later finite score moves it)
+  if constexpr (KS > 1) mrun = fmaxf(mrun, -1e30f);
 
   // tiles j with j + 1 < jfull: both S(j) and S(j+1) below the diagonal
   int j = 0;
@@ -415,7 +434,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   // the last tile (no S to start); a wave whose rows lie wholly before it skips it
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   __syncthreads();
-  if (q0 + 31 >= j * BN) {
+  if (q0 + 31 >= j * BN + kw) {
     u32x4 pk[2 * NB];
     pv_pre(Vbuf(j));
     softmax(sa, pk);
@@ -426,8 +445,74 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   // l of query c from lane c % 16 (register 0 for c < 16, 1 above)
   const float l_lo = __shfl(lsum[0], c & 15), l_hi = __shfl(lsum[1], c & 15);
   const float ltot = c < 16 ? l_lo : l_hi;
-  const float inv = 1.0f / ltot;
   uint16_t* orow = O + qbase + (size_t)m * D;
+  if constexpr (KS > 1) {
+    // Merge of a row's key groups.  O^T's accumulator is cut into pieces of PR registers
+    // (PR d values per lane), OWN pieces owned by each group: group i leaves (m_i, l_i) and
+    // the pieces it does not own in LDS, and a piece's owner adds all groups' to it, each
+    // scaled from its own reference point to M = max m_i.  Piece u of group i of row block
+    // wr: the 256 PR bytes from ((wr KS + i) NP + u) 256 PR, in 16-byte planes; (m_i, l_i)
+    // take the place of the first piece that i owns.
+    constexpr int PR = 2 * DB >= KS ? 8 : 4, NP = DB * 16 / PR, OWN = NP / KS, PB = 256 * PR;
+    static_assert(NP % KS == 0 && WR * KS * NP * PB <= 4 * TILE, "the pieces fit the tile buffers");
+    unsigned char* const rows = lds + wr * (KS * NP * PB);
+    auto ml_of = [&](int i) __attribute__((always_inline)) {
+      return reinterpret_cast<float*>(rows + (i * NP + i * OWN) * PB) + 2 * c;
+    };
+    __syncthreads();   // the last tile has been read
+    if (hh == 0) {
+      ml_of(kg)[0] = mrun;
+      ml_of(kg)[1] = ltot;
+    }
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      if (u / OWN != kg)
+#pragma unroll
+        for (int e = 0; e < PR; e += 4) {
+          const int db = u * PR / 16, g = u * PR % 16 + e;
+          *reinterpret_cast<f32x4*>(rows + (kg * NP + u) * PB + 256 * e + 16 * lane) =
+              f32x4{acc[db][g], acc[db][g + 1], acc[db][g + 2], acc[db][g + 3]};
+        }
+    __syncthreads();
+    float f[KS], l[KS], M = NEG_INF, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      l[i] = ml_of(i)[1];
+      f[i] = l[i] > 0.f ? ml_of(i)[0] : NEG_INF;   // (a group without a visible key counts for nothing)
+      M = fmaxf(M, f[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      f[i] = fast_exp2(f[i] - M);
+      L += f[i] * l[i];
+    }
+    const float inv = 1.0f / L;
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+      if (u / OWN == kg) {
+        const int db = u * PR / 16, g0 = u * PR % 16;
+        f32x16 x = f32x16{};
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+#pragma unroll
+          for (int e = 0; e < PR; e += 4) {
+            f32x4 y;
+            if (i == kg) y = f32x4{acc[db][g0 + e], acc[db][g0 + e + 1], acc[db][g0 + e + 2], acc[db][g0 + e + 3]};
+            else y = *reinterpret_cast<const f32x4*>(rows + (i * NP + u) * PB + 256 * e + 16 * lane);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) x[e + w] = __builtin_fmaf(f[i], y[w], x[e + w]);
+          }
+        const u32x4 o = pack8<E>(x, 0, inv);
+        uint16_t* const dst = orow + 32 * db + 16 * (g0 / 8) + 8 * hh + g0 % 8;
+        if (m < S) {
+          if constexpr (PR == 8) gstore16(dst, o);
+          else *reinterpret_cast<u32x2*>(dst) = u32x2{o[0], o[1]};
+        }
+      }
+    if (LSE && m < S && hh == 0 && kg == 0) Lse[(size_t)(b * H + hq) * S + m] = M + __log2f(L);
+    return;
+  }
+  const float inv = 1.0f / ltot;
   if (m < S) {  // rows of a partial last query tile past S are not stored
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
@@ -439,13 +524,16 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
 }
 
 // ---------------------------------------------------------------------------
-template <typename E, int D, int BM, int BN, int GH, bool LSE>
+template <typename E, int D, int BM, int BN, int GH, int KS, bool LSE>
 static int launch_fwd(const FwdArgs& a) {
-  constexpr int NT = 64 * (BM / 32) * GH;
+  constexpr int NT = 64 * (BM / 32) * GH * KS;
   const int total = a.B * (a.H / GH) * ((a.S + BM - 1) / BM);
-  hipLaunchKernelGGL((fwd_kernel<E, D, BM, BN, GH, LSE>), dim3(total), dim3(NT), 0, (hipStream_t)a.stream,
+  // (the 64 x 64 key-split workgroups run two per CU)
+  const int cus = KS == 2 ? cu_count() : 0;
+  const int first = total > cus && total <= 2 * cus ? cus : 0;
+  hipLaunchKernelGGL((fwd_kernel<E, D, BM, BN, GH, KS, LSE>), dim3(total), dim3(NT), 0, (hipStream_t)a.stream,
                      (const uint16_t*)a.q, (const uint16_t*)a.k, (const uint16_t*)a.v,
-                     (uint16_t*)a.o, a.lse, a.B, a.H, a.Hkv, a.S, a.scale_log2);
+                     (uint16_t*)a.o, a.lse, a.B, a.H, a.Hkv, a.S, a.scale_log2, first);
   return hipGetLastError() == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
 }
 
@@ -461,20 +549,28 @@ static int launch_fwd(const FwdArgs& a) {
 #define FA_FWD_PART 0
 #endif
 
-// Dispatch over the compile-time parameters of one (element type, D) slice.
+// Dispatch over the compile-time parameters of one (element type, D) slice; gh = -KS names
+// an instance of KS key groups.
 template <typename E, int D>
 static FwdFn pick_fwd(int bm, int bn, int gh, bool lse) {
 #define FA_CASE(BM_, BN_, GH_)                                                          \
   if (bm == BM_ && bn == BN_ && gh == GH_)                                             \
-    return lse ? launch_fwd<E, D, BM_, BN_, GH_, true> : launch_fwd<E, D, BM_, BN_, GH_, false>;
+    return lse ? launch_fwd<E, D, BM_, BN_, GH_, 1, true> : launch_fwd<E, D, BM_, BN_, GH_, 1, false>;
+#define FA_KEYS(BM_, BN_, KS_)                                                          \
+  if (bm == BM_ && bn == BN_ && gh == -KS_)                                            \
+    return lse ? launch_fwd<E, D, BM_, BN_, 1, KS_, true> : launch_fwd<E, D, BM_, BN_, 1, KS_, false>;
 #if FA_FWD_PART != 2
   FA_CASE(64, 64, 1) FA_CASE(64, 128, 1) FA_CASE(128, 64, 1) FA_CASE(128, 128, 1)
+  FA_KEYS(64, 64, 2)
+  if constexpr (D == 128) { FA_KEYS(64, 128, 4) }
+  else { FA_KEYS(32, 128, 4) }
 #endif
 #if FA_FWD_PART != 1
   FA_CASE(64, 64, 2) FA_CASE(64, 128, 2) FA_CASE(128, 64, 2)
   FA_CASE(64, 64, 4)
 #endif
 #undef FA_CASE
+#undef FA_KEYS
   return nullptr;
 }
 
@@ -485,7 +581,7 @@ static FwdFn pick_fwd(int bm, int bn, int gh, bool lse) {
 #if FA_FWD_PART == 1
 extern "C" FA_HIDDEN fa::FwdFn FA_FWD_TABLE_GROUPED(int bm, int bn, int gh, int lse);
 extern "C" FA_HIDDEN fa::FwdFn FA_FWD_TABLE(int bm, int bn, int gh, int lse) {
-  return gh == 1 ? fa::pick_fwd<FA_ETYPE, FA_D>(bm, bn, gh, lse != 0) : FA_FWD_TABLE_GROUPED(bm, bn, gh, lse);
+  return gh <= 1 ? fa::pick_fwd<FA_ETYPE, FA_D>(bm, bn, gh, lse != 0) : FA_FWD_TABLE_GROUPED(bm, bn, gh, lse);
 }
 #else
 extern "C" FA_HIDDEN fa::FwdFn FA_FWD_TABLE(int bm, int bn, int gh, int lse) {

@@ -63,7 +63,9 @@ enum fa_status {
  * block_m / block_n : query rows per head and keys per LDS tile, each in {64, 128}.
  *        block_m cannot change the result (each 32-row wave computes the same
  *        either way); where a 64-row single-head workgroup would leave SIMDs idle
- *        the library runs 128-row workgroups.
+ *        the library runs 128-row workgroups.  Up to three 64-row workgroups per CU
+ *        (B * H * ceil(S / 64)) the library splits each tile's keys over groups of
+ *        waves, in a shape of its own (fa_api.hip, fwd_key_split).
  *        S may be any length >= 1: a partial last query or key tile is masked (the
  *        reference requires S to be a multiple of both tiles, fused.py:70-71, and
  *        names partial edge tiles as future work).
@@ -164,7 +166,8 @@ FA_API size_t fa_noalloc_scratch_bytes(void);
  * fa_fwd_exact: fa_fwd with block_m query rows per head and heads_per_wg query heads
  *   (of one K/V group) per workgroup, block_n keys per tile.  FA_ERR_UNSUPPORTED when no
  *   kernel has that shape ((block_m, block_n, heads_per_wg) in {64,128}x{64,128}x{1},
- *   {64,128}x{64}x{2}, (64,128,2), (64,64,4)).
+ *   {64,128}x{64}x{2}, (64,128,2), (64,64,4)).  The range whose keys fa_fwd splits over
+ *   groups of waves is no choice of shape: there it runs fa_fwd's kernel (same results).
  * fa_bwd_gqa_exact: fa_bwd_gqa with the dQ kernel at dq_block_m x dq_block_n and the
  *   dK/dV key tiles split nsplit ways (1..64; > 1 needs a workspace of
  *   8*B*H*S (rounded up to 256) + 8*B*H_kv*nsplit*S*D bytes, else FA_ERR_WORKSPACE).
