@@ -4,8 +4,9 @@
 
 q, k, v: [B, H, N, D] float16 or bfloat16 GPU tensors.  Returns O with q's
 shape and dtype, enqueued on the current stream without synchronising (as the
-reference's ct.launch).  tile_m / tile_n select the kernel's query rows per
-workgroup and keys per LDS tile (each 64 or 128).  N may be any length: a
+reference's ct.launch).  tile_m / tile_n are the reference's tile arguments (each
+64 or 128), hints here: the library runs the workgroup shape that is fastest for
+the call.  N may be any length: a
 partial last tile is masked (the reference raises ValueError unless N is a
 multiple of both tiles, attention/fused/fused.py:70-71).
 """

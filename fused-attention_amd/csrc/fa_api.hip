@@ -151,6 +151,10 @@ bool fwd_key_split(int B, int H, int S, int D, FwdShape* out) {
 }
 
 int dq_block_m(int block_m, int /*D*/) { return block_m == 64 ? 128 : block_m; }
+// Keys per dQ tile (bitwise the same either way): at D = 128 a 128-key tile leaves one wave per
+// SIMD (backward, us of 128 / 64 keys: B=4 H=32 S=2048 579 / 520, B=2 H=16 H_kv=4 S=4096 499 / 470);
+// at D <= 64 both hold two, and 128 keys are 0-2 % faster.
+int dq_block_n(int block_n, int D) { return D == 128 ? 64 : block_n; }
 
 // Work items (key-tile chunks) the dK/dV kernel should have for its heavy-first order
 // to balance: two per workgroup slot the GPU holds at once, and one round more per
@@ -254,8 +258,12 @@ int fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   if (!q || !k || !v || !o) return FA_ERR_NULL;
   FwdShape w;
   if (!fwd_key_split(B, H, S, D, &w)) {
-    const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, block_n);
-    w = FwdShape{fwd_block_m(block_m, block_n, D, gh), block_n, gh};
+    // 64-key tiles whatever block_n: a 128-key tile needs more registers than two waves per
+    // SIMD have, and is slower everywhere (us of 128 x 128 / 128 x 64, D = 32, 64, 128: MHA B=4
+    // H=32 S=2048 89 / 62, 112 / 87, 189 / 139; GQA B=2 H=16 H_kv=4 S=4096 73 / 56, 97 / 77, 167 / 129;
+    // B=16 H=32 S=512 D=32 47 / 29)
+    const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, 64);
+    w = FwdShape{fwd_block_m(block_m, 64, D, gh), 64, gh};
   }
   fa::FwdFn fn = fwd_table(dtype, D, w.block_m, w.block_n, w.gh, lse != nullptr);
   if (!fn) return FA_ERR_UNSUPPORTED;
@@ -270,7 +278,7 @@ int fa_bwd(const void* q, const void* k, const void* v, const void* o,
   int st = check_common(B, H, S, D, dtype, block_m, block_n);
   if (st != FA_OK) return st;
   if (!q || !k || !v || !o || !d_o || !lse || !dq || !dk || !dv) return FA_ERR_NULL;
-  fa::BwdFn fn = bwd_table(dtype, D, dq_block_m(block_m, D), block_n);
+  fa::BwdFn fn = bwd_table(dtype, D, dq_block_m(block_m, D), dq_block_n(block_n, D));
   if (!fn) return FA_ERR_UNSUPPORTED;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H, S, D, scale_log2, sm_scale, hip_stream,
                 nullptr, nullptr, 1, nullptr, false};
@@ -292,7 +300,7 @@ int fa_bwd_gqa(const void* q, const void* k, const void* v, const void* o,
   if (H_kv <= 0 || H_kv > H || H % H_kv != 0) return FA_ERR_DIMS;
   if (!q || !k || !v || !o || !d_o || !lse || !dq || !dk || !dv) return FA_ERR_NULL;
   if (workspace && (reinterpret_cast<uintptr_t>(workspace) & 15)) return FA_ERR_WORKSPACE;
-  fa::BwdFn fn = bwd_table(dtype, D, dq_block_m(block_m, D), block_n);
+  fa::BwdFn fn = bwd_table(dtype, D, dq_block_m(block_m, D), dq_block_n(block_n, D));
   if (!fn) return FA_ERR_UNSUPPORTED;
   // the workspace holds, in this order and as far as it reaches: the per-row terms
   // (dQ then runs first and dK/dV reads Delta instead of forming it), then the

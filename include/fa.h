@@ -65,7 +65,9 @@ enum fa_status {
  *        either way); where a 64-row single-head workgroup would leave SIMDs idle
  *        the library runs 128-row workgroups.  Up to three 64-row workgroups per CU
  *        (B * H * ceil(S / 64)) the library splits each tile's keys over groups of
- *        waves, in a shape of its own (fa_api.hip, fwd_key_split).
+ *        waves, in a shape of its own (fa_api.hip, fwd_key_split).  block_n is a hint:
+ *        the library takes 64-key tiles where 128 would cost occupancy (the forward;
+ *        dQ at D = 128).
  *        S may be any length >= 1: a partial last query or key tile is masked (the
  *        reference requires S to be a multiple of both tiles, fused.py:70-71, and
  *        names partial edge tiles as future work).
@@ -173,7 +175,7 @@ FA_API size_t fa_noalloc_scratch_bytes(void);
  *   8*B*H*S (rounded up to 256) + 8*B*H_kv*nsplit*S*D bytes, else FA_ERR_WORKSPACE).
  *   A NULL workspace (nsplit 1) runs the dK/dV kernel that forms Delta in every key
  *   tile it meets, then dQ: the variant the row terms replace, kept for measurement.
- * The queries return what fa_fwd / fa_bwd_gqa choose for a shape (0: invalid).
+ * The queries return the rules' choice for a shape and tile (0: invalid).
  */
 FA_API int fa_fwd_exact(const void* q, const void* k, const void* v, void* o, float* lse,
                  int B, int H, int H_kv, int S, int D, int dtype, float scale_log2,
