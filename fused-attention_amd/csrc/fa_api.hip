@@ -211,6 +211,22 @@ int dkdv_nsplit(int B, int H, int H_kv, int S, int D) {
   return s < 1 ? 1 : (int)s;
 }
 
+// Whether the backward runs as bwd_small_kernel: dQ and dK/dV in one launch of 64-row and 64-key
+// workgroups (a split dK/dV keeps its kernel behind that launch's dQ).  By the number W of 64-row
+// workgroups: up to three per CU; at D = 128, whose workgroup has a CU to itself, one per CU.
+// Neither H_kv nor the workspace decides, so dQ is the same for all of them.
+// Measured, us of the two kernels / the one launch (W):
+//   D = 32:  B=2 H=8 S=1024 (256) 27.6 / 15.5, B=1 H=16 S=2240 (560) 52.6 / 42.0, B=3 H=8 S=2048 (768) 68.0 /
+//   51.1, B=8 H=16 S=512 (1024) 24.3 / 25.5
+//   D = 64:  B=2 H=8 S=512 (128) 23.4 / 12.2, B=2 H=16 S=1024 (512) 37.8 / 32.6, B=5 H=8 S=1000 (640) 52.5 /
+//   40.4, B=3 H=16 S=832 (624) 40.4 / 34.7, B=4 H=16 S=1024 (1024) 54.9 / 58.3
+//   D = 128: B=2 H=8 S=512 (128) 36.3 / 22.7, B=3 H=5 S=1000 (240) 56.5 / 46.3, B=2 H=8 S=1024 (256) 56.4 /
+//   45.2, B=3 H=8 S=768 (288) 47.2 / 47.8, B=4 H=16 S=512 (512) 39.9 / 59.0
+//   dQ alone of a split: B=1 H=4 S=4096 D=128 137 / 124, D=64 94 / 87; B=2 H=8 H_kv=2 S=2048 D=64 73 / 70
+bool bwd_small(int B, int H, int S, int D) {
+  return (long long)B * H * ((S + 63) / 64) <= (D == 128 ? 1LL : 3LL) * cu_count();
+}
+
 // ---------------------------------------------------------------------------
 // Device scratch of the allocation-free backward (fa_bwd_gqa_noalloc): stands in
 // for fa_bwd_gqa's caller workspace.  Each device that loads the library holds its
@@ -281,7 +297,7 @@ int fa_bwd(const void* q, const void* k, const void* v, const void* o,
   fa::BwdFn fn = bwd_table(dtype, D, dq_block_m(block_m, D), dq_block_n(block_n, D));
   if (!fn) return FA_ERR_UNSUPPORTED;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H, S, D, scale_log2, sm_scale, hip_stream,
-                nullptr, nullptr, 1, nullptr, false};
+                nullptr, nullptr, 1, nullptr, false, bwd_small(B, H, S, D)};
   return fn(a);
 }
 
@@ -318,7 +334,7 @@ int fa_bwd_gqa(const void* q, const void* k, const void* v, const void* o,
   float* wsk = nsplit > 1 ? reinterpret_cast<float*>(ws) : nullptr;
   float* wsv = nsplit > 1 ? wsk + (size_t)B * H_kv * nsplit * S * D : nullptr;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H_kv, S, D, scale_log2, sm_scale, hip_stream,
-                wsk, wsv, nsplit, rowb, false};
+                wsk, wsv, nsplit, rowb, false, bwd_small(B, H, S, D)};
   return fn(a);
 }
 
@@ -386,7 +402,7 @@ int fa_bwd_gqa_exact(const void* q, const void* k, const void* v, const void* o,
   float* wsk = nsplit > 1 ? reinterpret_cast<float*>(ws + rowb_bytes(B, H, S)) : nullptr;
   float* wsv = nsplit > 1 ? wsk + (size_t)B * H_kv * nsplit * S * D : nullptr;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H_kv, S, D, scale_log2, sm_scale, hip_stream,
-                wsk, wsv, nsplit, rowb, rowb == nullptr};
+                wsk, wsv, nsplit, rowb, rowb == nullptr, bwd_small(B, H, S, D)};
   return fn(a);
 }
 

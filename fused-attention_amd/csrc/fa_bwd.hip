@@ -4,7 +4,8 @@
 //   P  = exp2(S*c - LSE)     with S = Q K^T, c = log2(e)/sqrt(D), LSE from the forward
 //   dV = P^T dO              dP = dO V^T        Delta = rowsum(dO * O)
 //   dS = P * (dP - Delta)    dQ = dS K / sqrt(D)  dK = dS^T Q / sqrt(D)
-// Two kernels on the caller's stream: dK/dV then dQ, each forming Delta itself;
+// A grid that leaves the GPU idle runs as one launch (bwd_small_kernel, below).  Else
+// two kernels on the caller's stream: dK/dV then dQ, each forming Delta itself;
 // or, given a buffer for per-row terms, dQ first (it writes each query row's
 // -LSE/c and -Delta) and then dK/dV, which reads them instead of forming Delta.
 //   dkdv_kernel: one workgroup per key tile (128 keys, 32 per wave) of one K/V
@@ -35,6 +36,8 @@
 //                accumulates dQ^T += K^T dS^T, reading K^T with transposed reads.
 //                At D >= 64 the full tiles run a hand-pipelined schedule (operand
 //                reads two items ahead of their MFMAs).
+//   bwd_small_kernel: dQ and dK/dV together in 64-row and 64-key workgroups, two waves
+//                to every 32 rows or keys, for grids too small to fill the GPU.
 // No kernel uses atomics; each output element is written once.  Any S >= 1: the
 // last query and key tiles may be partial (rows past S read as zero, never stored).
 //
@@ -1568,6 +1571,387 @@ void dq_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
 }
 
 // ===========================================================================
+// Backward of a grid that leaves the GPU idle: dK / dV and dQ in one launch
+// ===========================================================================
+// Few heads or short sequences give the two kernels above fewer 128-row workgroups than the
+// GPU has CUs, and each waits for its longest chain of tiles.  Here both run in one
+// launch (neither waits for the other: dK/dV forms Delta itself), over tiles of 64 keys or 64
+// query rows, and two waves share every 32 of them: of each staged 64-row tile one takes the
+// first 32 rows and one the last, with accumulators of its own that are added through LDS at the
+// end.  A chain is then half as long per tile and the two kinds overlap; what it costs is twice
+// the staging per MFMA, so a grid that fills the GPU is slower this way (the rule and both
+// sides measured: fa_api.hip, bwd_small).
+// Workgroup wg < 2 min(nkv, ndq) is item wg / 2 of dK/dV (even) or of dQ (odd), the rest items of
+// the kind that is left; both kinds heaviest first.  nkv = 0: dQ alone (it then leaves the row
+// terms for a split dK/dV in Rb).
+template <int D>
+struct SmallBwd {
+  static constexpr int ROWB = 2 * D, TILE = 64 * ROWB, DB = D / 32;
+  static constexpr int OFF_L = 3 * TILE;                                // Q | dO | O | LSE
+  static constexpr int BUFA = OFF_L + 1024;
+  static constexpr int OFF_DELTA = 3 * BUFA, SMEM = OFF_DELTA + 2 * 64 * 4;
+  static_assert(4 * TILE <= SMEM, "dQ's double-buffered K and V tiles");
+  static_assert(4 * DB * 4096 <= SMEM, "the accumulators handed over at the end");
+};
+
+// DMA of one [64][D] tile, rows past `rows` zero: 4 waves, 1 KB blocks round-robin
+template <int D>
+struct SmallDma {
+  static constexpr int ROWB = 2 * D, CPR = ROWB / 16, NDMA = 64 * ROWB / 1024 / 4;
+  int vo[NDMA], wave;
+  __device__ __forceinline__ void init(int lane, int w) {
+    wave = w;
+#pragma unroll
+    for (int x = 0; x < NDMA; ++x) {
+      const int row = (w + 4 * x) * (1024 / ROWB) + lane / CPR;
+      vo[x] = row * ROWB + (((lane % CPR) ^ bswz(row, CPR)) << 4);
+    }
+  }
+  __device__ __forceinline__ void tile(const uint16_t* src, int rows, unsigned char* buf) const {
+    const auto rs = make_rsrc(src, rows * ROWB);
+#pragma unroll
+    for (int x = 0; x < NDMA; ++x) dma16(rs, buf + (wave + 4 * x) * 1024, vo[x], 0);
+  }
+};
+
+// A 32 x D accumulator in LDS, one 16-byte plane per 4 registers.
+template <int DB>
+__device__ __forceinline__ void acc_put(unsigned char* slot, const f32x16 (&a)[DB], int lane) {
+#pragma unroll
+  for (int i = 0; i < 4 * DB; ++i) {
+    const int g = 4 * (i & 3);
+    *reinterpret_cast<f32x4*>(slot + 1024 * i + 16 * lane) =
+        f32x4{a[i >> 2][g], a[i >> 2][g + 1], a[i >> 2][g + 2], a[i >> 2][g + 3]};
+  }
+}
+template <int DB>
+__device__ __forceinline__ void acc_add(const unsigned char* slot, f32x16 (&a)[DB], int lane) {
+#pragma unroll
+  for (int i = 0; i < 4 * DB; ++i) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(slot + 1024 * i + 16 * lane);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[i >> 2][4 * (i & 3) + e] += x[e];
+  }
+}
+
+template <typename E, int D>
+__device__ __forceinline__ void small_dq(unsigned char* lds, int item, const uint16_t* __restrict__ Q,
+                                         const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
+                                         const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO,
+                                         const float* __restrict__ Lse, uint16_t* __restrict__ dQ,
+                                         float* __restrict__ Rb, int B, int H, int Hkv, int S,
+                                         float scale_log2, float sm_scale) {
+  constexpr int ROWB = 2 * D, TILE = 64 * ROWB, KT = D / 16, DB = D / 32;
+  const float NEG_INF = -__builtin_inff();
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, hh = lane >> 5;
+  const int rb = wave & 1, kg = wave >> 1;   // 32-row block, and which 32 keys of every tile
+  const int nq = (S + 63) / 64;
+  const int bh = item % (B * H), qt = nq - 1 - item / (B * H);
+  const size_t base = (size_t)bh * S * D;
+  const size_t kvbase = (size_t)((bh / H) * Hkv + (bh % H) / (H / Hkv)) * S * D;
+  const int q0 = 64 * qt + 32 * rb, m = q0 + c, ntiles = qt + 1;
+
+  SmallDma<D> dma;
+  dma.init(lane, wave);
+  auto load = [&](int j, unsigned char* kb, unsigned char* vb) __attribute__((always_inline)) {
+    const int rows = min(64, S - 64 * j);
+    dma.tile(K + kvbase + (size_t)j * 64 * D, rows, kb);
+    dma.tile(V + kvbase + (size_t)j * 64 * D, rows, vb);
+  };
+  load(0, lds, lds + 2 * TILE);
+
+  u32x4 qf[KT], dof[KT];
+  float delta;
+  {
+    const size_t mr = base + (size_t)min(m, S - 1) * D + 8 * hh;   // rows >= S: any valid row, never stored
+    float part = 0.f;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      qf[t] = gload16(Q + mr + 16 * t);
+      dof[t] = gload16(dO + mr + 16 * t);
+      const u32x4 o = gload16(O + mr + 16 * t);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) part = dot_pair<E>(dof[t][w], o[w], part);
+    }
+    delta = halfwave_sum(part);
+  }
+  const float lse = Lse[(size_t)bh * S + min(m, S - 1)];
+  if (Rb != nullptr && kg == 0 && hh == 0 && m < S) {
+    const float inv_c = 1.0f / scale_log2;
+    Rb[(size_t)bh * S + m] = -lse * inv_c;
+    Rb[(size_t)B * H * S + (size_t)bh * S + m] = -delta;
+  }
+
+  TileOffsets<ROWB> to;
+  to.init(lane);
+  f32x16 acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) acc[db] = f32x16{};
+
+  auto block = [&](const unsigned char* ks, const unsigned char* vs, auto diag) __attribute__((always_inline)) {
+    f32x16 s = f32x16{}, dp = f32x16{};
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      s = mfma32<E>(lds_read16(ks, to.opnd[t]), qf[t], s);
+      dp = mfma32<E>(lds_read16(vs, to.opnd[t]), dof[t], dp);
+    }
+    float ds[16];
+#pragma unroll
+    for (int g = 0; g < 16; ++g) {
+      float x = s[g];
+      if (decltype(diag)::value && acc_row(g, hh) > c) x = NEG_INF;
+      ds[g] = fast_exp2(__builtin_fmaf(x, scale_log2, -lse)) * (dp[g] - delta);
+    }
+    u32x4 dsk[2];
+#pragma unroll
+    for (int i1 = 0; i1 < 2; ++i1)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) dsk[i1][q] = pack2<E>(ds[8 * i1 + 2 * q], ds[8 * i1 + 2 * q + 1]);
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i1 = 0; i1 < 2; ++i1)
+        acc[db] = mfma32<E>(tr_read2(ks, to.tr(db, i1, 0), to.tr(db, i1, 1)), dsk[i1], acc[db]);
+  };
+  // tile j in buffer j % 2 while tile j + 1 is in flight (the two buffers are restrict-qualified:
+  // the compiler need not wait for that DMA before the reads)
+  auto step = [&](int j, const unsigned char* __restrict__ kc, const unsigned char* __restrict__ vc,
+                  unsigned char* __restrict__ kn, unsigned char* __restrict__ vn) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(kBwdWaitVmcnt0);
+    __syncthreads();
+    if (j + 1 < ntiles) load(j + 1, kn, vn);
+    const int k0 = 64 * j + 32 * kg;
+    const unsigned char *ks = kc + 32 * kg * ROWB, *vs = vc + 32 * kg * ROWB;
+    if (k0 < q0) block(ks, vs, BTag<false>{});
+    else if (k0 == q0) block(ks, vs, BTag<true>{});
+  };
+  for (int j = 0; j < ntiles; ++j) {
+    const int p = j & 1;
+    step(j, lds + p * TILE, lds + (2 + p) * TILE, lds + (1 - p) * TILE, lds + (3 - p) * TILE);
+  }
+
+  // the two key groups' sums: each hands the other half of its pieces (8 registers) over
+  constexpr int NP = 2 * DB;
+  __syncthreads();
+  unsigned char* const slots = lds + rb * (2 * NP * 2048);
+#pragma unroll
+  for (int u = 0; u < NP; ++u)
+    if (u / DB != kg)
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const int g = 8 * (u & 1) + e;
+        *reinterpret_cast<f32x4*>(slots + (kg * NP + u) * 2048 + 256 * e + 16 * lane) =
+            f32x4{acc[u >> 1][g], acc[u >> 1][g + 1], acc[u >> 1][g + 2], acc[u >> 1][g + 3]};
+      }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NP; ++u)
+    if (u / DB == kg) {
+      f32x16 x = f32x16{};
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        const f32x4 y = *reinterpret_cast<const f32x4*>(slots + ((1 - kg) * NP + u) * 2048 + 256 * e + 16 * lane);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) x[e + w] = acc[u >> 1][8 * (u & 1) + e + w] + y[w];
+      }
+      if (m < S) gstore16(dQ + base + (size_t)m * D + 32 * (u >> 1) + 16 * (u & 1) + 8 * hh, pack8<E>(x, 0, sm_scale));
+    }
+}
+
+template <typename E, int D>
+__device__ __forceinline__ void small_dkdv(unsigned char* lds, int item, const uint16_t* __restrict__ Q,
+                                           const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
+                                           const uint16_t* __restrict__ O, const uint16_t* __restrict__ dO,
+                                           const float* __restrict__ Lse, uint16_t* __restrict__ dK,
+                                           uint16_t* __restrict__ dV, int B, int H, int Hkv, int S,
+                                           float scale_log2, float sm_scale) {
+  using SB = SmallBwd<D>;
+  constexpr int ROWB = 2 * D, CPR = ROWB / 16, TILE = 64 * ROWB, KT = D / 16, DB = D / 32;
+  const float NEG_INF = -__builtin_inff();
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, hh = lane >> 5;
+  const int kb = wave & 1, qg = wave >> 1;   // 32-key block, and which 32 rows of every query tile
+  const int G = H / Hkv, nq = (S + 63) / 64;
+  const int bkv = item % (B * Hkv), jt = item / (B * Hkv);
+  const size_t base = (size_t)bkv * S * D;
+  const int bh0 = (bkv / Hkv) * H + (bkv % Hkv) * G;   // first query head of the group
+  const int k0w = 64 * jt + 32 * kb, n = k0w + c;
+  const bool active = k0w < S;               // wave-uniform
+
+  // pair t: query tile jt + t / G of query head bh0 + t % G
+  const int T = G * (nq - jt);
+  SmallDma<D> dma;
+  dma.init(lane, wave);
+  int di = jt, dg = 0;   // the next pair to load
+  auto load = [&](unsigned char* buf) __attribute__((always_inline)) {
+    const size_t row0 = (size_t)(bh0 + dg) * S + (size_t)di * 64;
+    const int rows = min(64, S - di * 64);
+    dma.tile(Q + row0 * D, rows, buf);
+    dma.tile(dO + row0 * D, rows, buf + TILE);
+    dma.tile(O + row0 * D, rows, buf + 2 * TILE);
+    if (wave == 0) dma4(make_rsrc(Lse + row0, rows * 4), buf + SB::OFF_L, 4 * lane, 0);
+    if (++dg == G) {
+      dg = 0;
+      ++di;
+    }
+  };
+  auto bufp = [&](int t) __attribute__((always_inline)) {
+    return lds + __builtin_amdgcn_readfirstlane((t % 3) * SB::BUFA);
+  };
+  auto dlp = [&](int t) __attribute__((always_inline)) {
+    return reinterpret_cast<float*>(lds + SB::OFF_DELTA + (t & 1) * 256);
+  };
+  load(bufp(0));
+  if (T > 1) load(bufp(1));
+
+  u32x4 kf[KT], vf[KT];
+  if (active) {
+    const size_t nr = base + (size_t)min(n, S - 1) * D + 8 * hh;   // keys >= S: any valid row
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      kf[t] = gload16(K + nr + 16 * t);
+      vf[t] = gload16(V + nr + 16 * t);
+    }
+  }
+  TileOffsets<ROWB> to;
+  to.init(lane);
+  f32x16 dv_acc[DB], dk_acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) dv_acc[db] = dk_acc[db] = f32x16{};
+
+  // -Delta of a tile's rows into dl and -LSE / c in place (a lane quad per row)
+  const float inv_c = 1.0f / scale_log2;
+  auto row_terms = [&](unsigned char* buf, float* dl) __attribute__((always_inline)) {
+    const int row = tid / 4, part = tid % 4;
+    float a = 0.f;
+#pragma unroll
+    for (int x = 0; x < CPR / 4; ++x) {
+      const int off = row * ROWB + (((part + 4 * x) ^ bswz(row, CPR)) << 4);
+      const u32x4 d = lds_read16(buf + TILE, off), o = lds_read16(buf + 2 * TILE, off);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) a = dot_pair<E>(d[w], o[w], a);
+    }
+    a = quad_sum(a);
+    float* ls = reinterpret_cast<float*>(buf + SB::OFF_L);
+    const float l = -ls[row] * inv_c;
+    dl[row] = -a;
+    ls[row] = l;
+  };
+  auto rows16 = [&](const float* src) __attribute__((always_inline)) {
+    f32x16 v;
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(src + 32 * qg + 8 * gq + 4 * hh);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * gq + e] = x[e];
+    }
+    return v;
+  };
+  auto block = [&](const unsigned char* buf, const float* dl, auto diag) __attribute__((always_inline)) {
+    f32x16 s = rows16(reinterpret_cast<const float*>(buf + SB::OFF_L)), dp = rows16(dl);
+    const unsigned char *qs = buf + 32 * qg * ROWB, *dos = qs + TILE;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      s = mfma32<E>(lds_read16(qs, to.opnd[t]), kf[t], s);
+      dp = mfma32<E>(lds_read16(dos, to.opnd[t]), vf[t], dp);
+    }
+    u32x4 pk[2], dsk[2];
+    float p[16], ds[16];
+#pragma unroll
+    for (int g = 0; g < 16; ++g) {
+      float x = s[g];
+      if (decltype(diag)::value && c > acc_row(g, hh)) x = NEG_INF;
+      p[g] = fast_exp2(x * scale_log2);
+      ds[g] = p[g] * dp[g];
+    }
+#pragma unroll
+    for (int i1 = 0; i1 < 2; ++i1)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        pk[i1][q] = pack2<E>(p[8 * i1 + 2 * q], p[8 * i1 + 2 * q + 1]);
+        dsk[i1][q] = pack2<E>(ds[8 * i1 + 2 * q], ds[8 * i1 + 2 * q + 1]);
+      }
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i1 = 0; i1 < 2; ++i1) {
+        dv_acc[db] = mfma32<E>(tr_read2(dos, to.tr(db, i1, 0), to.tr(db, i1, 1)), pk[i1], dv_acc[db]);
+        dk_acc[db] = mfma32<E>(tr_read2(qs, to.tr(db, i1, 0), to.tr(db, i1, 1)), dsk[i1], dk_acc[db]);
+      }
+  };
+
+  __builtin_amdgcn_s_waitcnt(kBwdWaitVmcnt0);
+  __syncthreads();
+  row_terms(bufp(0), dlp(0));
+  // pair t in buffer t % 3 while pair t + 1 has landed (its row terms are formed) and pair
+  // t + 2 is in flight
+  auto step = [&](int t, unsigned char* __restrict__ cur, unsigned char* __restrict__ nxt,
+                  unsigned char* __restrict__ dst, const float* __restrict__ dl, float* __restrict__ dln)
+      __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(kBwdWaitVmcnt0);
+    __syncthreads();
+    if (t + 2 < T) load(dst);
+    const int q0 = 64 * (jt + t / G) + 32 * qg;   // this wave's first query row
+    if (active) {
+      if (q0 > k0w) block(cur, dl, BTag<false>{});
+      else if (q0 == k0w) block(cur, dl, BTag<true>{});
+    }
+    if (t + 1 < T) row_terms(nxt, dln);
+  };
+  for (int t = 0; t < T; ++t) step(t, bufp(t), bufp(t + 1), bufp(t + 2), dlp(t), dlp(t + 1));
+
+  // the two query groups' sums: group 0 stores dV, group 1 dK
+  __syncthreads();
+  unsigned char* const slot = lds + kb * (2 * DB * 4096);
+  if (qg == 0) acc_put(slot, dk_acc, lane);
+  else acc_put(slot + DB * 4096, dv_acc, lane);
+  __syncthreads();
+  if (qg == 0) acc_add(slot + DB * 4096, dv_acc, lane);
+  else acc_add(slot, dk_acc, lane);
+  if (n >= S) return;
+  uint16_t* const r = (qg ? dK : dV) + base + (size_t)n * D + 8 * hh;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i1 = 0; i1 < 2; ++i1)
+      gstore16(r + db * 32 + 16 * i1,
+               qg ? pack8<E>(dk_acc[db], 8 * i1, sm_scale) : pack8<E>(dv_acc[db], 8 * i1, 1.0f));
+}
+
+template <typename E, int D>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(D == 128 ? 1 : 2, D == 128 ? 1 : 2)))
+void bwd_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
+                      const uint16_t* __restrict__ V, const uint16_t* __restrict__ O,
+                      const uint16_t* __restrict__ dO, const float* __restrict__ Lse,
+                      uint16_t* __restrict__ dQ, uint16_t* __restrict__ dK, uint16_t* __restrict__ dV,
+                      float* __restrict__ Rb, int B, int H, int Hkv, int S, float scale_log2, float sm_scale,
+                      int nkv, int ndq) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[SmallBwd<D>::SMEM];
+  const int wg = blockIdx.x, pairs = min(nkv, ndq);
+  const bool paired = wg < 2 * pairs;
+  const bool kv = paired ? (wg & 1) == 0 : nkv > ndq;
+  const int item = paired ? wg >> 1 : wg - pairs;
+  if (kv) small_dkdv<E, D>(lds, item, Q, K, V, O, dO, Lse, dK, dV, B, H, Hkv, S, scale_log2, sm_scale);
+  else small_dq<E, D>(lds, item, Q, K, V, O, dO, Lse, dQ, Rb, B, H, Hkv, S, scale_log2, sm_scale);
+}
+
+// dQ, and dK / dV unless `dkdv` is false.
+template <typename E, int D>
+static bool launch_small(const BwdArgs& a, bool dkdv) {
+  const int nt = (a.S + 63) / 64;
+  const int nkv = dkdv ? a.B * a.Hkv * nt : 0, ndq = a.B * a.H * nt;
+  hipLaunchKernelGGL((bwd_small_kernel<E, D>), dim3(nkv + ndq), dim3(256), 0, (hipStream_t)a.stream,
+                     (const uint16_t*)a.q, (const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.o,
+                     (const uint16_t*)a.d_o, a.lse, (uint16_t*)a.dq, (uint16_t*)a.dk, (uint16_t*)a.dv, a.rowb,
+                     a.B, a.H, a.Hkv, a.S, a.scale_log2, a.sm_scale, nkv, ndq);
+  return hipGetLastError() == hipSuccess;
+}
+
+// ===========================================================================
 // dK / dV from per-chunk partial sums
 // ===========================================================================
 // dK[bkv, n, :] = sum over c < nsplit of Pk[bkv * nsplit + c, n, :] (and dV from
@@ -1716,6 +2100,11 @@ static bool launch_dq(const BwdArgs& a) {
 // Without one, dK/dV runs first and forms Delta from O and dO in every workgroup.
 template <typename E, int D, int BMQ, int BNK>
 static int launch_bwd(const BwdArgs& a) {
+  if (a.small) {
+    if (a.nsplit <= 1) return launch_small<E, D>(a, true) ? FA_OK : FA_ERR_LAUNCH;
+    // (a split has the row terms' buffer)
+    return launch_small<E, D>(a, false) && launch_dkdv<E, D, 64, 128>(a) ? FA_OK : FA_ERR_LAUNCH;
+  }
   if (a.rowb) {
     if (!launch_dq<E, D, BMQ, BNK>(a)) return FA_ERR_LAUNCH;
     return launch_dkdv<E, D, 64, 128>(a) ? FA_OK : FA_ERR_LAUNCH;

@@ -46,6 +46,8 @@ struct BwdArgs {
   // last), or, with form_delta, formed by the dK/dV kernel in every key tile
   float* rowb;
   bool form_delta;
+  // the grid leaves the GPU idle: dQ, and dK / dV where it is not split, in one launch
+  bool small;
 };
 
 // keys per dK/dV workgroup (4 waves x 32 keys), for the split heuristics on the host

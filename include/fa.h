@@ -84,7 +84,9 @@ FA_API int fa_fwd(const void* q, const void* k, const void* v, void* o, float* l
  * workgroup per key tile) reads them, then dQ (one workgroup per query tile) forms
  * its own and overwrites dq.  No workspace.  When dq is not 16-byte aligned the
  * dK/dV kernel forms Delta from the O and dO tiles of every key tile instead (same
- * results up to the fp32 summation order of Delta, slower).
+ * results up to the fp32 summation order of Delta, slower).  Small grids (up to three
+ * 64-row workgroups per CU, one at D = 128) run as one launch that forms Delta itself
+ * and leaves dq to dQ alone (fa_api.hip, bwd_small).
  *
  * Replaces attention/backward/fused_backward.py:173-184 (_backward: the torch
  * Delta op at :175 and the two launches at :180-183).
@@ -173,6 +175,8 @@ FA_API size_t fa_noalloc_scratch_bytes(void);
  * fa_bwd_gqa_exact: fa_bwd_gqa with the dQ kernel at dq_block_m x dq_block_n and the
  *   dK/dV key tiles split nsplit ways (1..64; > 1 needs a workspace of
  *   8*B*H*S (rounded up to 256) + 8*B*H_kv*nsplit*S*D bytes, else FA_ERR_WORKSPACE).
+ *   On grids that fa_bwd_gqa runs as one launch, dQ (and an unsplit dK/dV) are that
+ *   launch's here too.
  *   A NULL workspace (nsplit 1) runs the dK/dV kernel that forms Delta in every key
  *   tile it meets, then dQ: the variant the row terms replace, kept for measurement.
  * The queries return the rules' choice for a shape and tile (0: invalid).
