@@ -167,10 +167,30 @@ def check_tiles(tile_m, tile_n):
         raise ValueError(f"tile_m={tile_m} and tile_n={tile_n} must each be 64 or 128")
 
 
+_forward = None
+
+
+def _forward_op():
+    """The C++ module's forward; False where only libfa.so is built or FA_LIB_PATH names another
+    library (the module links the one beside it): the same C entry is then called through ctypes."""
+    global _forward
+    if _forward is None:
+        try:
+            _forward = "FA_LIB_PATH" not in os.environ and autograd().forward
+        except LibraryError:
+            load()  # (raises if the library itself is absent)
+            _forward = False
+    return _forward
+
+
 def fwd(q, k, v, o, lse, tile_m, tile_n):
     """Enqueue the forward on the current stream.  Shapes already checked by the caller."""
-    lib = load()
+    op = _forward or _forward_op()
     _require_device(q, k, v, o)
+    if op:
+        check(op(q, k, v, o, lse, dtype_code(q.dtype), int(tile_m), int(tile_n)), "fa_fwd")
+        return
+    lib = load()
     B, H, S, D = q.shape
     H_kv = k.shape[1]
     code = lib.fa_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse),
