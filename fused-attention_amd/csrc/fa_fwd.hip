@@ -80,7 +80,8 @@ constexpr float kSumLimit = float(1 << FA_RESCALE_THRESHOLD);
 
 template <int D, int BM, int BN, int GH, int KS>
 constexpr int fwd_waves_per_simd() {
-  return (BN / KS <= 64 && (BM / 32) * GH * KS >= 4) ? 2 : 1;
+  // (64 rows of one head, two waves: at D = 128 its LDS allows one wave per SIMD anyway)
+  return (BN / KS <= 64 && ((BM / 32) * GH * KS >= 4 || D <= 64)) ? 2 : 1;
 }
 
 // Compile-time marker of a pipeline iteration that runs wholly below the diagonal.

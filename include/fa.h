@@ -63,7 +63,8 @@ enum fa_status {
  * block_m / block_n : query rows per head and keys per LDS tile, each in {64, 128}.
  *        block_m cannot change the result (each 32-row wave computes the same
  *        either way); where a 64-row single-head workgroup would leave SIMDs idle
- *        the library runs 128-row workgroups.  Up to three 64-row workgroups per CU
+ *        the library runs 128-row workgroups, or, for short sequences at D <= 64, 64-row ones
+ *        whatever block_m.  Up to three 64-row workgroups per CU
  *        (B * H * ceil(S / 64)) the library splits each tile's keys over groups of
  *        waves, in a shape of its own (fa_api.hip, fwd_key_split).  block_n is a hint:
  *        the library takes 64-key tiles where 128 would cost occupancy (the forward;
@@ -179,7 +180,9 @@ FA_API size_t fa_noalloc_scratch_bytes(void);
  *   launch's here too.
  *   A NULL workspace (nsplit 1) runs the dK/dV kernel that forms Delta in every key
  *   tile it meets, then dQ: the variant the row terms replace, kept for measurement.
- * The queries return the rules' choice for a shape and tile (0: invalid).
+ * The queries return the rules' choice for a shape and tile (0: invalid); the two row
+ *   queries, which take no length, that of sequences past the short ones (fa_api.hip,
+ *   short_rows).
  */
 FA_API int fa_fwd_exact(const void* q, const void* k, const void* v, void* o, float* lse,
                  int B, int H, int H_kv, int S, int D, int dtype, float scale_log2,
