@@ -104,7 +104,7 @@ HEADER = [
     "\"Occupancy\" is the compiler's waves per SIMD for the registers and LDS; \"Scheduler\" the machine",
     "scheduler options its object is built under (the Makefile's `SCHED_*`: strategy, pre-RA direction).",
     "Template arguments:",
-    "`fwd_kernel<E, D, rows per head, keys per tile, heads per workgroup, LSE>`,",
+    "`fwd_kernel<E, D, rows per head, keys per tile, heads per workgroup, key groups, LSE>`,",
     "`dq_kernel<E, D, rows, keys>`, `dkdv_kernel<E, D, query rows per tile, keys per workgroup, per-row terms>`,",
     "`dkdv_pair_kernel<E, D, query rows per tile, keys per workgroup>` (D = 128 only).",
     "",
