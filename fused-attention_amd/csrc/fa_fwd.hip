@@ -126,7 +126,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, hh = lane >> 5;
-  const int wh = wave % GH, wr = wave / GH % WR;
+  const int wh = wave % GH, wr = KS > 1 ? wave % WR : wave / GH;
   const int kg = KS > 1 ? wave / WR : 0;   // this wave's key group
   const int kw = kg * (32 * NB);           // and its first key in a tile
 
