@@ -405,8 +405,7 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
     body(j, Kbuf(j + 1), Kbuf(j), Vbuf(j), Vbuf(j + 1), sc, sn, st);
   };
 
-  // prologue: K(0), V(0), K(1) in flight; S(0) and its row max, the first reference
-  // point (key 0 lies at or below every row, so the max is finite)
+  // prologue: K(0), V(0), K(1) in flight; S(0) and its row max, the first reference point
   dma_k(0, Kbuf(0));
   dma_v(0, Vbuf(0));
   if (ntiles > 1) dma_k(1, Kbuf(1));
@@ -415,10 +414,10 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   f32x16 sa[NB], sb[NB];
   s_tile(Kbuf(0), sa);
   if (jfull == 0) mask_tile(sa, 0);
-  mrun = tile_max(sa);
-  // (a key group that meets no key of its rows in tile 0 has no finite score: a finite
-  // reference point keeps its P at zero, and a later finite score moves it)
-  if constexpr (KS > 1) mrun = fmaxf(mrun, -1e30f);
+  // (a row whose scores in tile 0 are all -inf, the keys masked by the caller or, with key groups,
+  // none of this group's at or below the row: the least finite reference point keeps its P at zero,
+  // and any later score moves it)
+  mrun = fmaxf(tile_max(sa), -__FLT_MAX__);
 
   // tiles j with j + 1 < jfull: both S(j) and S(j+1) below the diagonal
   int j = 0;

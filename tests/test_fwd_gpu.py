@@ -132,6 +132,25 @@ def test_forward_lse(dt, tiles):
     assert torch.equal(o, fused_attention(q, k, v, *tiles))
 
 
+@pytest.mark.parametrize("tiles", TILES, ids=lambda t: f"{t[0]}x{t[1]}")
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_leading_keys_of_minus_infinite_score(D, tiles):
+    """Keys 0..63 score -inf in every row (left padding masked by the caller): the rows past them
+    are the attention over the other keys, whatever the tile (160 heads keep the call off the
+    kernels that split keys over wave groups).  Beside the fp32 formula, with the suites' bars."""
+    g = torch.Generator(device="cuda").manual_seed(D + sum(tiles))
+    q, k, v = (torch.randn(1, 160, 300, D, device="cuda", generator=g).bfloat16() for _ in range(3))
+    q[..., 0] = 1.0
+    k[:, :, :64, 0] = float("-inf")
+    out, lse = _forward(q, k, v, *tiles)
+    s = (q.float() @ k.float().transpose(-1, -2).contiguous()) / math.sqrt(D)
+    s.masked_fill_(torch.triu(torch.ones(300, 300, device="cuda", dtype=torch.bool), 1), float("-inf"))
+    want = torch.softmax(s, -1) @ v.float()
+    assert torch.isfinite(out[:, :, 64:]).all()
+    assert bool(((out.float() - want).abs() <= 2e-2 + 2e-2 * want.abs())[:, :, 64:].all())
+    assert float((lse - torch.logsumexp(s, -1) * LOG2E)[:, :, 64:].abs().max()) <= LSE_ABS["bf16"]
+
+
 def test_non_default_stream_and_repeatability():
     B, H, N, D = 1, 4, 1024, 128
     q, k, v = (dev(x, torch.bfloat16) for x in cases.normal_inputs([(B, H, N, D)] * 3, seed=5))
