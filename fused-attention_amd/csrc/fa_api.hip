@@ -391,8 +391,6 @@ int fa_fwd_exact(const void* q, const void* k, const void* v, void* o, float* ls
   if (!q || !k || !v || !o) return FA_ERR_NULL;
   fa::FwdFn fn = fwd_table(dtype, D, block_m, block_n, heads_per_wg, lse != nullptr);
   if (!fn) return FA_ERR_UNSUPPORTED;
-  FwdShape w;
-  if (fwd_key_split(B, H, S, D, &w)) fn = fwd_table(dtype, D, w.block_m, w.block_n, w.gh, lse != nullptr);
   fa::FwdArgs a{q, k, v, o, lse, B, H, H_kv, S, D, scale_log2, hip_stream};
   return fn(a);
 }
@@ -420,7 +418,7 @@ int fa_bwd_gqa_exact(const void* q, const void* k, const void* v, const void* o,
   float* wsk = nsplit > 1 ? reinterpret_cast<float*>(ws + rowb_bytes(B, H, S)) : nullptr;
   float* wsv = nsplit > 1 ? wsk + (size_t)B * H_kv * nsplit * S * D : nullptr;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H_kv, S, D, scale_log2, sm_scale, hip_stream,
-                wsk, wsv, nsplit, rowb, rowb == nullptr, bwd_small(B, H, S, D)};
+                wsk, wsv, nsplit, rowb, rowb == nullptr, false};
   return fn(a);
 }
 

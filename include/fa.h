@@ -171,13 +171,13 @@ FA_API size_t fa_noalloc_scratch_bytes(void);
  * fa_fwd_exact: fa_fwd with block_m query rows per head and heads_per_wg query heads
  *   (of one K/V group) per workgroup, block_n keys per tile.  FA_ERR_UNSUPPORTED when no
  *   kernel has that shape ((block_m, block_n, heads_per_wg) in {64,128}x{64,128}x{1},
- *   {64,128}x{64}x{2}, (64,128,2), (64,64,4)).  The range whose keys fa_fwd splits over
- *   groups of waves is no choice of shape: there it runs fa_fwd's kernel (same results).
+ *   {64,128}x{64}x{2}, (64,128,2), (64,64,4)).  Keys are never split over groups of waves
+ *   here: where fa_fwd does so this is the kernel it does not take (results equal up to the
+ *   rounding of P against other reference points).
  * fa_bwd_gqa_exact: fa_bwd_gqa with the dQ kernel at dq_block_m x dq_block_n and the
  *   dK/dV key tiles split nsplit ways (1..64; > 1 needs a workspace of
  *   8*B*H*S (rounded up to 256) + 8*B*H_kv*nsplit*S*D bytes, else FA_ERR_WORKSPACE).
- *   On grids that fa_bwd_gqa runs as one launch, dQ (and an unsplit dK/dV) are that
- *   launch's here too.
+ *   Always the two kernels, also on grids that fa_bwd_gqa runs as one launch.
  *   A NULL workspace (nsplit 1) runs the dK/dV kernel that forms Delta in every key
  *   tile it meets, then dQ: the variant the row terms replace, kept for measurement.
  * The queries return the rules' choice for a shape and tile (0: invalid); the two row
