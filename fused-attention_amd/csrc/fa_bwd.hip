@@ -2100,26 +2100,25 @@ static bool launch_dq(const BwdArgs& a) {
 // Without one, dK/dV runs first and forms Delta from O and dO in every workgroup.
 template <typename E, int D, int BMQ, int BNK>
 static int launch_bwd(const BwdArgs& a) {
-  if (a.small) {
-    if (a.nsplit <= 1) return launch_small<E, D>(a, true) ? FA_OK : FA_ERR_LAUNCH;
-    // (a split has the row terms' buffer)
-    return launch_small<E, D>(a, false) && launch_dkdv<E, D, 64, 128>(a) ? FA_OK : FA_ERR_LAUNCH;
-  }
+  if (a.small && a.nsplit <= 1) return launch_small<E, D>(a, true) ? FA_OK : FA_ERR_LAUNCH;
+  const auto dq = a.small ? [](const BwdArgs& x) { return launch_small<E, D>(x, false); } : launch_dq<E, D, BMQ, BNK>;
   if (a.rowb) {
-    if (!launch_dq<E, D, BMQ, BNK>(a)) return FA_ERR_LAUNCH;
+    if (!dq(a)) return FA_ERR_LAUNCH;
     return launch_dkdv<E, D, 64, 128>(a) ? FA_OK : FA_ERR_LAUNCH;
   }
   // dK/dV first: dQ's own output buffer holds the per-row terms until dQ, which runs
   // last and forms its own, overwrites it (8 bytes per row in a 2 D-byte row).  With
   // form_delta (the study entry's variant) dK/dV forms them in every key tile instead.
+  // (A small grid comes here with a split whose sums fit a workspace too short for the
+  // row terms: more than 2 D query heads to a K/V head.)
   if (!a.form_delta && (reinterpret_cast<uintptr_t>(a.dq) & 15) == 0) {
     BwdArgs t = a;
     t.rowb = static_cast<float*>(a.dq);
     if (!launch_rowterms<E, D>(t, t.rowb) || !launch_dkdv<E, D, 64, 128>(t)) return FA_ERR_LAUNCH;
-    return launch_dq<E, D, BMQ, BNK>(a) ? FA_OK : FA_ERR_LAUNCH;
+    return dq(a) ? FA_OK : FA_ERR_LAUNCH;
   }
   if (!launch_dkdv<E, D, 64, 128>(a)) return FA_ERR_LAUNCH;
-  return launch_dq<E, D, BMQ, BNK>(a) ? FA_OK : FA_ERR_LAUNCH;
+  return dq(a) ? FA_OK : FA_ERR_LAUNCH;
 }
 
 template <typename E, int D>

@@ -87,3 +87,35 @@ def test_entries_agree(Hkv, S, D):
                 assert torch.equal(g, r)
             else:
                 assert float((g.float() - r.float()).abs().max()) <= 2e-2 + 1e-2 * float(r.float().abs().max())
+
+
+def test_split_without_room_for_the_row_terms():
+    """128 query heads to one K/V head at D = 32: a workspace 256 bytes short of the row terms (8 bytes
+    per query row) still holds the sums of a three-way split (8 D bytes per key and chunk).  Same
+    gradients, bitwise, as with the row terms in the workspace before the same split; with dq 8
+    bytes off its alignment dK/dV forms Delta itself, in another fp32 order."""
+    lib = _lib.load()
+    H, S, D = 128, 100, 32
+    q, k, v, do = make(1, H, 1, S, D, torch.float16, seed=7)
+    o, lse = _forward(q, k, v, 64, 64)
+    rows, chunk = 8 * H * S, 8 * S * D
+    assert rows % 256 == 0 and rows - 256 >= 3 * chunk and lib.fa_bwd_dkdv_split(1, H, 1, S, D) > 3
+
+    def run(nbytes, off=0):
+        dq = torch.zeros(q.numel() + 16, device="cuda", dtype=q.dtype)[off:off + q.numel()]
+        dk, dv = torch.zeros_like(k), torch.zeros_like(v)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        code = lib.fa_bwd_gqa(*(ctypes.c_void_p(t.data_ptr()) for t in (q, k, v, o, do, lse, dq, dk, dv)), 1, H, 1, S, D,
+                              _lib.dtype_code(q.dtype), _lib.scale_log2(D), 1.0 / math.sqrt(D), 64, 64, _lib._ptr(ws),
+                              nbytes, _lib._stream(q.device))
+        _lib.check(code, "fa_bwd_gqa")
+        torch.cuda.synchronize()
+        return dq, dk, dv
+
+    want = run(rows + 3 * chunk)
+    for got, want_t in zip(run(rows - 256), want):
+        assert torch.equal(got, want_t)
+    dq, dk, dv = run(rows - 256, off=4)
+    assert torch.equal(dq, want[0])
+    for got, want_t in ((dk, want[1]), (dv, want[2])):   # sums over 128 heads: a few fp16 units
+        assert float((got.float() - want_t.float()).abs().max()) <= 8 * 2.0 ** -10 * float(want_t.float().abs().max())
