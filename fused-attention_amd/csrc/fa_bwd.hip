@@ -1939,15 +1939,15 @@ void bwd_small_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict
   else small_dq<E, D>(lds, item, Q, K, V, O, dO, Lse, dQ, Rb, B, H, Hkv, S, scale_log2, sm_scale);
 }
 
-// dQ, and dK / dV unless `dkdv` is false.
+// dQ, and dK / dV unless `dkdv` is false (then the row terms too, where there is a buffer for them).
 template <typename E, int D>
 static bool launch_small(const BwdArgs& a, bool dkdv) {
   const int nt = (a.S + 63) / 64;
   const int nkv = dkdv ? a.B * a.Hkv * nt : 0, ndq = a.B * a.H * nt;
   hipLaunchKernelGGL((bwd_small_kernel<E, D>), dim3(nkv + ndq), dim3(256), 0, (hipStream_t)a.stream,
                      (const uint16_t*)a.q, (const uint16_t*)a.k, (const uint16_t*)a.v, (const uint16_t*)a.o,
-                     (const uint16_t*)a.d_o, a.lse, (uint16_t*)a.dq, (uint16_t*)a.dk, (uint16_t*)a.dv, a.rowb,
-                     a.B, a.H, a.Hkv, a.S, a.scale_log2, a.sm_scale, nkv, ndq);
+                     (const uint16_t*)a.d_o, a.lse, (uint16_t*)a.dq, (uint16_t*)a.dk, (uint16_t*)a.dv,
+                     dkdv ? nullptr : a.rowb, a.B, a.H, a.Hkv, a.S, a.scale_log2, a.sm_scale, nkv, ndq);
   return hipGetLastError() == hipSuccess;
 }
 

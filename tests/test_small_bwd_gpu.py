@@ -119,3 +119,23 @@ def test_split_without_room_for_the_row_terms():
     assert torch.equal(dq, want[0])
     for got, want_t in ((dk, want[1]), (dv, want[2])):   # sums over 128 heads: a few fp16 units
         assert float((got.float() - want_t.float()).abs().max()) <= 8 * 2.0 ** -10 * float(want_t.float().abs().max())
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_one_launch_leaves_the_workspace_alone(D):
+    """Both kinds of workgroup of the one launch form Delta themselves: nothing reads row terms, so
+    none are written into the workspace a caller gives."""
+    lib = _lib.load()
+    B, H, S = 1, 3, 200
+    q, k, v, do = make(B, H, H, S, D, torch.float16, seed=D)
+    o, lse = _forward(q, k, v, 64, 64)
+    assert lib.fa_bwd_dkdv_split(B, H, H, S, D) == 1
+    n = lib.fa_bwd_gqa_workspace_size(B, H, H, S, D)
+    ws = torch.full((n,), 0xA5, dtype=torch.uint8, device="cuda")
+    grads = [torch.empty_like(t) for t in (q, k, v)]
+    code = lib.fa_bwd_gqa(*(ctypes.c_void_p(t.data_ptr()) for t in (q, k, v, o, do, lse, *grads)), B, H, H, S, D,
+                          _lib.dtype_code(q.dtype), _lib.scale_log2(D), 1.0 / math.sqrt(D), 64, 64, _lib._ptr(ws), n,
+                          _lib._stream(q.device))
+    _lib.check(code, "fa_bwd_gqa")
+    torch.cuda.synchronize()
+    assert bool((ws == 0xA5).all())
