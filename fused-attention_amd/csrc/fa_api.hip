@@ -426,7 +426,8 @@ int fa_fwd_heads_per_wg(int B, int H, int H_kv, int S, int D, int block_m, int b
   if (B <= 0 || H <= 0 || S <= 0 || H_kv <= 0 || H_kv > H || H % H_kv != 0) return 0;
   if (D != 32 && D != 64 && D != 128) return 0;
   if (!tile_ok(block_m) || !tile_ok(block_n)) return 0;
-  return fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, block_n);
+  if (fwd_key_split(B, H, S, D, nullptr)) return 1;
+  return fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, 64);   // (fa_fwd's tiles are 64 keys whatever block_n)
 }
 
 int fa_fwd_rows_per_wg(int block_m, int block_n, int D, int heads_per_wg) {

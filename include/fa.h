@@ -180,9 +180,10 @@ FA_API size_t fa_noalloc_scratch_bytes(void);
  *   Always the two kernels, also on grids that fa_bwd_gqa runs as one launch.
  *   A NULL workspace (nsplit 1) runs the dK/dV kernel that forms Delta in every key
  *   tile it meets, then dQ: the variant the row terms replace, kept for measurement.
- * The queries return the rules' choice for a shape and tile (0: invalid); the two row
- *   queries, which take no length, that of sequences past the short ones (fa_api.hip,
- *   short_rows).
+ * The queries return the rules' choice for a shape and tile (0: invalid): heads_per_wg 1
+ *   also where the one head's keys are split over groups of waves; the two row queries, which
+ *   take neither a length nor a grid, the rows of full grids past the short sequences
+ *   (fa_api.hip, fwd_key_split, bwd_small and short_rows).
  */
 FA_API int fa_fwd_exact(const void* q, const void* k, const void* v, void* o, float* lse,
                  int B, int H, int H_kv, int S, int D, int dtype, float scale_log2,

@@ -231,13 +231,17 @@ def test_exact_shape_entries_and_rule_queries(lib):
     assert lib.fa_fwd_heads_per_wg(2, 32, 8, 8192, 128, 128, 64) == 4   # 128-row tile as four 64-row heads
     assert lib.fa_fwd_rows_per_wg(128, 64, 128, 4) == 64
     assert lib.fa_fwd_heads_per_wg(1, 32, 1, 16384, 64, 128, 64) == 4
-    assert lib.fa_fwd_heads_per_wg(2, 8, 1, 2048, 128, 128, 64) == 2    # four would leave CUs short
-    assert lib.fa_fwd_heads_per_wg(2, 8, 1, 1024, 128, 64, 64) == 2   # 4 -> 2: under 2 workgroups per CU
+    assert lib.fa_fwd_heads_per_wg(2, 16, 4, 2048, 128, 128, 64) == 2   # four would leave CUs short
+    assert lib.fa_fwd_heads_per_wg(2, 16, 4, 2048, 128, 64, 64) == 2  # 4 -> 2: under 2 workgroups per CU
+    assert lib.fa_fwd_heads_per_wg(2, 8, 1, 2048, 128, 128, 64) == 1    # one head, keys split over waves
+    assert lib.fa_fwd_heads_per_wg(2, 8, 1, 1024, 128, 64, 64) == 1
     assert lib.fa_fwd_heads_per_wg(1, 16, 4, 4096, 128, 64, 64) == 2  # one per CU at four heads
     assert lib.fa_fwd_heads_per_wg(2, 8, 1, 8192, 128, 64, 64) == 4   # two per CU: four stay
     assert lib.fa_fwd_heads_per_wg(2, 8, 1, 8192, 64, 64, 64) == 4
     assert lib.fa_fwd_heads_per_wg(2, 8, 1, 8192, 32, 64, 64) == 2    # D = 32: under 4 per CU
-    assert lib.fa_fwd_heads_per_wg(1, 32, 1, 16384, 64, 64, 128) == 2
+    assert lib.fa_fwd_heads_per_wg(1, 32, 1, 16384, 64, 64, 128) == 4   # 128-key tiles run as 64-key ones
+    assert lib.fa_fwd_heads_per_wg(2, 32, 8, 8192, 128, 64, 128) == 4
+    assert lib.fa_fwd_heads_per_wg(2, 32, 8, 8192, 128, 128, 128) == 4
     # dK/dV split: two items per workgroup slot (the paired D = 128 kernel one slot per CU, the
     # one-wave kernel two), one round more per 8192 keys; no split under 64 pairs per key tile
     assert lib.fa_bwd_dkdv_split(4, 32, 32, 4096, 128) == 1
