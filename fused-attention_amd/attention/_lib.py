@@ -171,14 +171,15 @@ _forward = None
 
 
 def _forward_op():
-    """The C++ module's forward; False where only libfa.so is built or FA_LIB_PATH names another
-    library (the module links the one beside it): the same C entry is then called through ctypes."""
+    """The C++ module's forward; False where there is none beside the library that is loaded (only
+    libfa.so is built, the module is of a build without it, or FA_LIB_PATH named another library:
+    the module links the one beside it): the same C entry is then called through ctypes."""
     global _forward
     if _forward is None:
+        load()  # (raises if the library itself is absent)
         try:
-            _forward = "FA_LIB_PATH" not in os.environ and autograd().forward
+            _forward = LIB_PATH == os.path.join(_PKG_ROOT, "libfa.so") and getattr(autograd(), "forward", False)
         except LibraryError:
-            load()  # (raises if the library itself is absent)
             _forward = False
     return _forward
 

@@ -163,3 +163,23 @@ def test_autograd_node_loads_without_a_gpu():
     mod = _lib.autograd()
     assert callable(mod.fused_attention)
     assert _lib.autograd() is mod
+
+
+@pytest.mark.parametrize("case", ["other library", "older module", "no module", "beside"])
+def test_forward_op_belongs_to_the_loaded_library(monkeypatch, case):
+    """The C++ module links the library beside it: its forward is taken only if that one is loaded,
+    and a module without it (of an older build, or none) leaves the ctypes call."""
+    from attention import _lib
+    _lib.load()
+    monkeypatch.setattr(_lib, "_forward", None)
+    monkeypatch.delenv("FA_LIB_PATH", raising=False)
+    monkeypatch.setattr(_lib, "LIB_PATH", _lib._PKG_ROOT + "/libfa.so")
+
+    def missing():
+        raise _lib.LibraryError("not built")
+    op = object()
+    monkeypatch.setattr(_lib, "autograd", {"older module": lambda: object(), "no module": missing}.get(
+        case, lambda: type("M", (), {"forward": op})))
+    if case == "other library":   # FA_LIB_PATH was set when this module was imported, and no longer is
+        monkeypatch.setattr(_lib, "LIB_PATH", "/elsewhere/libfa.so")
+    assert _lib._forward_op() is (op if case == "beside" else False)
