@@ -120,19 +120,32 @@ int fwd_block_m(int block_m, int /*block_n*/, int /*D*/, int gh) {
   if (gh == 4) return 64;  // four heads run 64-row tiles (fwd_heads_per_wg)
   return (block_m == 64 && gh == 1) ? 128 : block_m;
 }
-// Short sequences at D <= 64: one-head forward workgroups and dQ workgroups of 64 rows (two waves,
-// two to three per SIMD) in place of 128.  With so few key tiles a workgroup is mostly start, diagonal
-// and tail: smaller ones overlap them better, and half as many rows past S and masked tiles
-// are computed (most where ceil(S / 64) is odd).  Longer rows want the 128 that share a staged tile.
+// Short sequences at D <= 64: one-head forward workgroups and dQ workgroups of 64 rows (two waves)
+// in place of 128.  With so few key tiles a workgroup is mostly start, diagonal and tail: smaller ones
+// overlap them better, and half as many rows past S and masked tiles are computed (most where
+// ceil(S / 64) is odd).  They stage K and V twice as often, though.  Past three tiles that pays only
+// where the heads are a multiple of 8, so that each XCD finds its own heads' keys in its L2 and
+// no other's; past seven (D = 32: eight) also only where the 128-row workgroups are more
+// than two and a half per CU, below which they start all at once or nearly (four and a half at D = 64
+// with an even number of tiles, whose last 128-row workgroups are full).
 // Measured, us of 128 / 64 rows (bitwise equal):
-//   forward D = 32: B=16 H=32 S=200 12.7 / 11.4, S=512 28.4 / 25.8, S=576 36.1 / 30.2, S=700 46.4 / 39.5; B=4 H=16
-//   S=900 13.8 / 12.2; B=8 H=16 S=1024 20.9 / 22.2; B=3 H=16 S=1500 17.0 / 19.4
-//   forward D = 64: B=16 H=32 S=384 26.3 / 25.1, S=576 48.3 / 42.8, S=700 65.0 / 58.4; B=4 H=16 S=900 18.2 /
-//   16.4; B=8 H=16 S=1024 28.3 / 30.9; B=3 H=16 S=1500 23.8 / 27.2; up to two 64-row workgroups per CU
-//   128 rows stay (B=8 H=16 S=256 7.2 / 7.6, D = 32 5.9 / 6.1)
+//   forward D = 32: B=16 H=32 S=200 12.7 / 11.4, S=512 28.4 / 25.8, S=576 36.1 / 30.2, S=700 46.4 / 39.5;
+//   B=8 H=16 S=1024 20.9 / 22.2; B=3 H=16 S=1500 17.0 / 19.4
+//   forward D = 64: B=16 H=32 S=384 26.3 / 25.1, S=576 48.3 / 42.8, S=700 65.0 / 58.4; B=8 H=16 S=1024 28.3 /
+//   30.9; B=3 H=16 S=1500 23.8 / 27.2; up to two 64-row workgroups per CU 128 rows stay (B=8 H=16
+//   S=256 7.2 / 7.6, D = 32 5.9 / 6.1); 258 heads S=192 11.7 / 11.1, but past it, no multiple of 8: 133
+//   heads S=384 10.3 / 12.8, 341 heads S=768 48.7 / 71.4, 585 heads S=896 97.3 / 157.5; and few 128-row
+//   workgroups: 72 heads S=768 14.0 / 15.5, 96 heads S=705 14.5 / 16.3, 256 heads S=512 21.1 / 21.9
 //   backward (dQ at 64 rows) D = 32 / 64: B=16 H=32 S=256 33.1 / 32.1, 52.7 / 51.5; B=16 H=32 S=576 87.2 / 82.3,
-//   139 / 132; B=8 H=16 S=700 42.6 / 39.5, 64.9 / 60.0; B=8 H=16 S=1100 71.8 / 73.4, 106 / 107
-bool short_rows(int S, int D) { return D <= 64 && S <= 960; }
+//   139 / 132; B=8 H=16 S=700 42.6 / 39.5, 64.9 / 60.0; 341 heads S=768 91.5 / 97.1, 141 / 163; 72 heads S=768
+//   D = 32 26.5 / 28.3; B=8 H=16 S=1100 71.8 / 73.4, 106 / 107
+bool short_rows(int B, int H, int S, int D) {
+  if (D > 64 || S <= 192) return D <= 64;
+  const long long heads = (long long)B * H;
+  if (heads % 8 != 0 || S > 960) return false;
+  const bool full = D == 64 && (S + 63) / 64 % 2 == 0;
+  return S <= (D == 32 ? 512 : 448) || 2 * heads * ((S + 127) / 128) > (full ? 9LL : 5LL) * cu_count();
+}
 // Forward instance of a call.  Below a grid that fills the GPU the keys of a tile are split
 // over groups of waves (fwd_kernel's KS): the call then waits for the serial chain of the
 // last rows, and every other CU, or SIMD of a CU, idles.  By the number W of 64-row
@@ -168,8 +181,8 @@ int dq_block_m(int block_m, int /*D*/) { return block_m == 64 ? 128 : block_m; }
 // SIMD (backward, us of 128 / 64 keys: B=4 H=32 S=2048 579 / 520, B=2 H=16 H_kv=4 S=4096 499 / 470);
 // at D <= 64 both hold two, and 128 keys are 0-2 % faster.
 int dq_block_n(int block_n, int D) { return D == 128 ? 64 : block_n; }
-fa::BwdFn bwd_fn(int dtype, int D, int S, int block_m, int block_n) {
-  if (short_rows(S, D)) return bwd_table(dtype, D, 64, 64);
+fa::BwdFn bwd_fn(int dtype, int D, int B, int H, int S, int block_m, int block_n) {
+  if (short_rows(B, H, S, D)) return bwd_table(dtype, D, 64, 64);
   return bwd_table(dtype, D, dq_block_m(block_m, D), dq_block_n(block_n, D));
 }
 
@@ -296,7 +309,7 @@ int fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     // H=32 S=2048 89 / 62, 112 / 87, 189 / 139; GQA B=2 H=16 H_kv=4 S=4096 73 / 56, 97 / 77, 167 / 129;
     // B=16 H=32 S=512 D=32 47 / 29)
     const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, 64);
-    const bool few = gh == 1 && short_rows(S, D) && (long long)B * H * ((S + 63) / 64) > 2LL * cu_count();
+    const bool few = gh == 1 && short_rows(B, H, S, D) && (long long)B * H * ((S + 63) / 64) > 2LL * cu_count();
     w = FwdShape{few ? 64 : fwd_block_m(block_m, 64, D, gh), 64, gh};
   }
   fa::FwdFn fn = fwd_table(dtype, D, w.block_m, w.block_n, w.gh, lse != nullptr);
@@ -312,7 +325,7 @@ int fa_bwd(const void* q, const void* k, const void* v, const void* o,
   int st = check_common(B, H, S, D, dtype, block_m, block_n);
   if (st != FA_OK) return st;
   if (!q || !k || !v || !o || !d_o || !lse || !dq || !dk || !dv) return FA_ERR_NULL;
-  fa::BwdFn fn = bwd_fn(dtype, D, S, block_m, block_n);
+  fa::BwdFn fn = bwd_fn(dtype, D, B, H, S, block_m, block_n);
   if (!fn) return FA_ERR_UNSUPPORTED;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H, S, D, scale_log2, sm_scale, hip_stream,
                 nullptr, nullptr, 1, nullptr, false, bwd_small(B, H, S, D)};
@@ -334,7 +347,7 @@ int fa_bwd_gqa(const void* q, const void* k, const void* v, const void* o,
   if (H_kv <= 0 || H_kv > H || H % H_kv != 0) return FA_ERR_DIMS;
   if (!q || !k || !v || !o || !d_o || !lse || !dq || !dk || !dv) return FA_ERR_NULL;
   if (workspace && (reinterpret_cast<uintptr_t>(workspace) & 15)) return FA_ERR_WORKSPACE;
-  fa::BwdFn fn = bwd_fn(dtype, D, S, block_m, block_n);
+  fa::BwdFn fn = bwd_fn(dtype, D, B, H, S, block_m, block_n);
   if (!fn) return FA_ERR_UNSUPPORTED;
   // the workspace holds, in this order and as far as it reaches: the per-row terms
   // (dQ then runs first and dK/dV reads Delta instead of forming it), then the

@@ -2,7 +2,8 @@
 
 A 32-row wave does the same work in a workgroup of any size, so O, LSE and the gradients must equal,
 bitwise, those of the exact entry points at 128 rows.  Lengths: one key tile and one row past it,
-an odd and an even number of 64-row tiles, both sides of the rule's last length; every grid is
+an odd and an even number of 64-row tiles; both sides of each bound of the rule (three tiles; seven
+or eight; heads a multiple of 8; two and a half or four and a half 128-row workgroups per CU; 15 tiles); every grid is
 past those whose keys are split over wave groups."""
 
 import pytest
@@ -16,7 +17,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("B,H,H_kv,S,D,dtype", [
     (16, 32, 32, 65, 64, torch.float16), (16, 32, 32, 129, 32, torch.bfloat16), (16, 20, 4, 192, 64, torch.bfloat16),
-    (4, 17, 17, 960, 32, torch.float16), (4, 17, 17, 960, 64, torch.bfloat16), (4, 16, 16, 961, 64, torch.float16),
+    (2, 99, 99, 193, 32, torch.float16), (2, 100, 100, 256, 64, torch.bfloat16), (8, 16, 16, 448, 64, torch.float16),
+    (8, 16, 16, 449, 64, torch.bfloat16), (8, 16, 16, 512, 32, torch.float16), (8, 16, 16, 513, 32, torch.bfloat16),
+    (2, 44, 44, 960, 32, torch.float16), (2, 44, 44, 960, 64, torch.bfloat16), (2, 40, 40, 960, 64, torch.float16),
+    (2, 44, 44, 961, 64, torch.float16), (8, 36, 36, 449, 64, torch.float16), (16, 19, 19, 512, 64, torch.bfloat16),
 ])
 def test_short_rows_equal_128_rows(B, H, H_kv, S, D, dtype):
     lib = _lib.load()
