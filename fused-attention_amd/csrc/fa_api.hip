@@ -152,25 +152,44 @@ bool short_rows(int B, int H, int S, int D) {
 // workgroups, which depends on neither tile_m nor H_kv (results still depend on neither):
 //   W <= one per CU:  D <= 64: 32 rows x 4 groups over 128-key tiles; D = 128, whose 128-key
 //     tiles allow one workgroup per CU: 64 rows x 4 groups
-//   W <= three per CU, S >= 512 (below, a chain is a few tiles and the merge costs as much:
-//     B=16 H=32 S=64 D=64 5.2 -> 5.4 us, B=16 H=8 S=384 D=128 15.3 -> 15.5): 64 rows x 2 groups
-//     over 64-key tiles (D = 128 at S >= 4096 and W <= two per CU: 64 x 4 again)
-// Measured, us of unsplit / 64 x 2 / 64 x 4 / 32 x 4 (x: not an instance):
+//   W <= three per CU: 64 rows x 2 groups over 64-key tiles (D = 128 at S >= 4096 and W <= two per
+//     CU: 64 x 4 again)
+// A chain must be long enough to pay for the merge and for workgroups of half the rows, which
+// stage K and V twice as often; the more workgroups, the longer.  Where the heads are no multiple
+// of 8 the XCDs share them, each staging every shared head's keys through its own L2, which the
+// extra staging pays for again: at an odd number of heads each of the 8 streams all.
+// Measured, us of unsplit / 64 x 2 / 64 x 4 / 32 x 4:
 //   D = 64:  B=2 H=8 S=512 (W = 128) 8.6 / 6.6 / 6.9 / 5.8; B=8 H=1 S=1755 (224) 18.7 / 13.4 / 11.8 /
 //   10.8; B=1 H=2 S=8192 (256) 68.8 / 48.3 / 36.9 / 34.5; B=2 H=8 S=2048 (512) 21.5 / 16.2 / 17.8 / 19.0;
 //   B=2 H=16 S=1024 (512) 13.2 / 9.9 / 13.4 / 13.3
 //   D = 128: B=3 H=5 S=1000 (240) 17.6 / 15.0 / 15.1 / 17.8; B=1 H=1 S=16384 (256) 201 / 153 / 120 / 119;
 //   B=2 H=8 S=2048 (512) 31.2 / 28.1 / 28.0 / 43.7; B=1 H=8 S=4096 (512) 56.2 / 49.7 / 44.3 / 68.0;
 //   GQA B=1 H=32 H_kv=8 S=1531 (768) 30.1 / 27.9 / 36.0 / 55.6; B=2 H=16 S=2048 (1024) 41.9 / 44.1 / 54 / 88
-//   and through this rule, us before / after: D = 32: B=2 H=8 S=512 7.3 / 5.4, S=1024 10.8 / 6.0, B=1 H=4
-//   S=4096 31.2 / 13.9, B=2 H=8 S=2048 18.0 / 12.4; B=3 H=8 S=2048 (768): D = 32 25.2 / 16.1, D = 64
-//   32.6 / 21.9, D = 128 46.7 / 34.9; B=3 H=16 S=1024 (768): D = 64 19.7 / 16.1, D = 128 27.8 / 23.5
+// and the lengths from which the split pays, us of unsplit / split (heads of all batches, W; graph
+// replays, without the launches; at about 4000 sizes, groups of 1 to 32, the split calls now lie between
+// 0.29 and 1.03 of the unsplit ones, mean 0.81):
+//   W <= half the CUs: D = 64 S=64, 128 heads 4.20 / 4.41, S=100, 64 heads 5.21 / 4.46
+//   W <= one per CU: D = 64 S=64, 256 heads 4.39 / 5.33, GQA S=100, 128 heads 4.96 / 5.33, S=256, 64 heads 0.82 of it;
+//   D = 128: S=64, 128 heads 5.27 / 7.07, S=128, 128 heads 6.89 / 7.59, S=320 1.07, S=384, 42 heads 10.47 / 10.29
+//   W <= two: D = 64 S=512, 64 heads 9.66 / 7.56, MQA 19 / 12; D = 128 S=640, 48 heads 14.7 / 12.8, 51 heads
+//   15.9 / 16.6, S=1024, 25 heads 19.8 / 17.6
+//   W <= two and a half: D = 64 S=640, GQA, 64 heads 10.1 / 10.9, S=896, 45 heads 15.0 / 13.7; D = 128 S=833, 45
+//   heads 20.9 / 24.2, S=1280, 32 heads 26.6 / 22.9, 31 heads 26.2 / 28.1
+//   W <= three: GQA D = 64 S=640, 76 heads 10.6 / 12.5, S=1024, 48 heads 18.6 / 14.7, 44 heads 14.7 / 15.1, S=1531, 31
+//   heads 21.2 / 19.0; D = 128 S=1024, 48 heads 27.3 / 22.8, 46 heads 24.8 / 26.3, S=1531, 31 heads 32.2 / 36.4
 struct FwdShape {
   int block_m, block_n, gh;   // gh = -KS: key groups
 };
 bool fwd_key_split(int B, int H, int S, int D, FwdShape* out) {
-  const long long w = (long long)B * H * ((S + 63) / 64), cus = cu_count();
-  if (w > 3 * cus || (w > cus && S < 512)) return false;
+  const long long heads = (long long)B * H, w = heads * ((S + 63) / 64), cus = cu_count();
+  int past;   // the longest S that is not split
+  if (2 * w <= cus) past = D == 128 ? 320 : 64;
+  else if (w <= cus) past = D == 128 ? 320 : 128;
+  else if (w <= 2 * cus) past = D < 128 || heads % 4 == 0 ? 511 : 896;
+  else if (2 * w <= 5 * cus) past = D < 128 || heads % 2 == 0 ? 832 : 1400;
+  else if (w <= 3 * cus && (D < 128 || heads % 2 == 0)) past = heads % 8 == 0 ? 832 : 1280;
+  else return false;
+  if (S <= past) return false;
   const bool four = w <= cus || (D == 128 && S >= 4096 && w <= 2 * cus);
   if (out) *out = !four ? FwdShape{64, 64, -2} : D == 128 ? FwdShape{64, 128, -4} : FwdShape{32, 128, -4};
   return true;

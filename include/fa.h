@@ -65,8 +65,9 @@ enum fa_status {
  *        either way); where a 64-row single-head workgroup would leave SIMDs idle
  *        the library runs 128-row workgroups, or, for short sequences at D <= 64, 64-row ones
  *        whatever block_m.  Up to three 64-row workgroups per CU
- *        (B * H * ceil(S / 64)) the library splits each tile's keys over groups of
- *        waves, in a shape of its own (fa_api.hip, fwd_key_split).  block_n is a hint:
+ *        (B * H * ceil(S / 64)), and from a length on that grows with them, the library
+ *        splits each tile's keys over groups of waves, in a shape of its own (fa_api.hip,
+ *        fwd_key_split).  block_n is a hint:
  *        the library takes 64-key tiles where 128 would cost occupancy (the forward;
  *        dQ at D = 128).
  *        S may be any length >= 1: a partial last query or key tile is masked (the
