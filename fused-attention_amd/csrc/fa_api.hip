@@ -262,18 +262,29 @@ int dkdv_nsplit(int B, int H, int H_kv, int S, int D) {
 
 // Whether the backward runs as bwd_small_kernel: dQ and dK/dV in one launch of 64-row and 64-key
 // workgroups (a split dK/dV keeps its kernel behind that launch's dQ).  By the number W of 64-row
-// workgroups: up to three per CU; at D = 128, whose workgroup has a CU to itself, one per CU.
+// workgroups: at D = 128, whose workgroup has a CU to itself, up to one per CU; at D <= 64 up to two and
+// a half or three.  Less for short sequences: with one or two tiles to a chain there is
+// little to halve and the two launches are already short, so the twofold staging decides sooner.
 // Neither H_kv nor the workspace decides, so dQ is the same for all of them.
 // Measured, us of the two kernels / the one launch (W):
 //   D = 32:  B=2 H=8 S=1024 (256) 27.6 / 15.5, B=1 H=16 S=2240 (560) 52.6 / 42.0, B=3 H=8 S=2048 (768) 68.0 /
-//   51.1, B=8 H=16 S=512 (1024) 24.3 / 25.5
-//   D = 64:  B=2 H=8 S=512 (128) 23.4 / 12.2, B=2 H=16 S=1024 (512) 37.8 / 32.6, B=5 H=8 S=1000 (640) 52.5 /
-//   40.4, B=3 H=16 S=832 (624) 40.4 / 34.7, B=4 H=16 S=1024 (1024) 54.9 / 58.3
+//   51.1, B=8 H=16 S=512 (1024) 24.3 / 25.5; 381 heads S=128 (762) 12.9 / 13.9, MQA 128 heads S=384 (768) 46.3 / 49.3
+//   D = 64:  B=2 H=8 S=512 (128) 23.4 / 12.2, B=2 H=16 S=1024 (512) 37.8 / 32.6, B=3 H=16 S=832 (624) 40.4 /
+//   34.7, B=4 H=16 S=1024 (1024) 54.9 / 58.3; 512 heads S=64 (512) 13.0 / 14.8, 251 heads S=128 (502) 15.4 /
+//   17.1, 384 heads S=128 (768) 20.5 / 23.5, 125 heads S=320 (625) 24.1 / 25.3, 75 heads S=600 (750) 35.3 / 38.0,
+//   16 heads S=3000 (752) 103 / 109
 //   D = 128: B=2 H=8 S=512 (128) 36.3 / 22.7, B=3 H=5 S=1000 (240) 56.5 / 46.3, B=2 H=8 S=1024 (256) 56.4 /
-//   45.2, B=3 H=8 S=768 (288) 47.2 / 47.8, B=4 H=16 S=512 (512) 39.9 / 59.0
+//   45.2, B=3 H=8 S=768 (288) 47.2 / 47.8, B=4 H=16 S=512 (512) 39.9 / 59.0; 256 heads S=64 (256) 15.3 / 20.1, 128
+//   heads S=64 (128) 0.67 of the two kernels
 //   dQ alone of a split: B=1 H=4 S=4096 D=128 137 / 124, D=64 94 / 87; B=2 H=8 H_kv=2 S=2048 D=64 73 / 70
+// At about 3900 sizes, groups of 1 to 32, the calls that take it lie between 0.44 and 1.03 of the
+// two kernels' time, mean 0.74.
 bool bwd_small(int B, int H, int S, int D) {
-  return (long long)B * H * ((S + 63) / 64) <= (D == 128 ? 1LL : 3LL) * cu_count();
+  int quarters;   // of a 64-row workgroup per CU
+  if (D == 128) quarters = S <= 64 ? 2 : 4;
+  else if (D == 64) quarters = S <= 48 ? 12 : S <= 64 ? 6 : S <= 128 ? 7 : S <= 384 ? 9 : S <= 640 ? 10 : 11;
+  else quarters = S <= 384 ? 10 : 12;
+  return 4LL * B * H * ((S + 63) / 64) <= (long long)quarters * cu_count();
 }
 
 // ---------------------------------------------------------------------------

@@ -86,8 +86,8 @@ FA_API int fa_fwd(const void* q, const void* k, const void* v, void* o, float* l
  * workgroup per key tile) reads them, then dQ (one workgroup per query tile) forms
  * its own and overwrites dq.  No workspace.  When dq is not 16-byte aligned the
  * dK/dV kernel forms Delta from the O and dO tiles of every key tile instead (same
- * results up to the fp32 summation order of Delta, slower).  Small grids (up to three
- * 64-row workgroups per CU, one at D = 128) run as one launch that forms Delta itself
+ * results up to the fp32 summation order of Delta, slower).  Small grids (up to two
+ * to three 64-row workgroups per CU, one at D = 128) run as one launch that forms Delta itself
  * and leaves dq to dQ alone (fa_api.hip, bwd_small).
  *
  * Replaces attention/backward/fused_backward.py:173-184 (_backward: the torch

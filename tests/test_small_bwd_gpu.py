@@ -2,7 +2,7 @@
 keys), and the two-kernel backward and unsplit forward just past them.
 
 The one launch takes up to three 64-row workgroups per CU (256 CUs: B * H * ceil(S / 64) <= 768),
-one at D = 128; the forward splits keys over waves up to three, below 512 rows up to one.
+one at D = 128, fewer for short sequences.
 Lengths sit at the edges of the 32-row halves and the 64-row tiles; head counts put the grid just
 inside or just past the rule, so ragged lengths meet both kernels.  Bars of the backward suites
 (tests/test_gqa_bwd_gpu.py: check)."""
@@ -17,6 +17,7 @@ from attention import _lib
 from attention.backward.fused_backward import _forward
 from tests.gpu_util import log
 from tests.test_gqa_bwd_gpu import check, make
+from test_exact_entries_gpu import bwd
 
 pytestmark = pytest.mark.gpu
 
@@ -50,6 +51,27 @@ def test_ragged_lengths_past_the_rule(S, D):
 def test_edges_of_the_rule(B, H, Hkv, S, D):
     q, k, v, do = make(B, H, Hkv, S, D, MANY_HEADS, seed=B + H + S)
     check(q, k, v, do, (128, 64), f"small bwd edge B{B} H{H}/{Hkv} S{S} D{D}")
+
+
+# (heads, S, D, one launch): both sides of each bound
+ROUTES = [(128, 64, 128, True), (129, 64, 128, False), (128, 128, 128, True), (129, 100, 128, False),
+          (768, 48, 64, True), (769, 48, 64, False), (384, 64, 64, True), (385, 64, 64, False),
+          (224, 128, 64, True), (225, 128, 64, False), (144, 256, 64, True), (145, 256, 64, False),
+          (64, 640, 64, True), (65, 640, 64, False), (64, 704, 64, True), (65, 704, 64, False),
+          (106, 384, 32, True), (107, 384, 32, False), (109, 448, 32, True), (110, 448, 32, False)]
+
+
+@pytest.mark.parametrize("H,S,D,one", ROUTES)
+def test_where_the_backward_is_one_launch(H, S, D, one):
+    """Calls that the one launch makes slower run the two kernels: bitwise the exact entry's, which always
+    does.  A call of one launch differs from it by the fp32 summation order somewhere."""
+    lib = _lib.load()
+    q, k, v, do = make(1, H, H, S, D, MANY_HEADS, seed=H + S)
+    o, lse = _forward(q, k, v, 64, 64)
+    assert lib.fa_bwd_dkdv_split(1, H, H, S, D) == 1
+    got = bwd(lib, q, k, v, o, do, lse, 64, 64)
+    want = bwd(lib, q, k, v, o, do, lse, 64, 64, nsplit=1)
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) is not one
 
 
 @pytest.mark.parametrize("Hkv,S,D", [(4, 1000, 128), (1, 1200, 64), (4, 4200, 64)])
