@@ -6,7 +6,8 @@ Forward  = the fused forward kernel with the LSE output switched on: it writes
            lse = m + log2(l) (base-2 log-sum-exp of the scores pre-multiplied by
            log2(e)/sqrt(D)) directly, where the reference stores m and l and adds
            them with a torch op (:61-62, :169).
-Backward = two atomic-free kernels on the same stream:
+Backward = two atomic-free kernels on the same stream (one launch of both, each forming Delta,
+           where the grid leaves the GPU idle):
   dQ kernel:    one workgroup per query tile; loops over the visible key tiles;
                 dQ = scale * dS K.  Forms Delta = rowsum(dO * O) from the O and dO
                 rows it holds in registers (the reference runs it as a separate torch

@@ -106,7 +106,9 @@ HEADER = [
     "Template arguments:",
     "`fwd_kernel<E, D, rows per head, keys per tile, heads per workgroup, key groups, LSE>`,",
     "`dq_kernel<E, D, rows, keys>`, `dkdv_kernel<E, D, query rows per tile, keys per workgroup, per-row terms>`,",
-    "`dkdv_pair_kernel<E, D, query rows per tile, keys per workgroup>` (D = 128 only).",
+    "`dkdv_pair_kernel<E, D, query rows per tile, keys per workgroup>` (D = 128 only),",
+    "`bwd_small_kernel<E, D>` (dQ and dK/dV of small grids).  Each forward and dQ instance names its waves per SIMD",
+    "as minimum and maximum, so an occupancy of 2 may stand beside registers that allow 3.",
     "",
 ]
 

@@ -47,7 +47,8 @@ fa::BwdFn bwd_table(int dtype, int D, int bm, int bn) {
 // Query heads per workgroup for a GQA group: as many heads of one K/V group
 // as fit in 8 waves (512 threads), each head taking block_m/32 waves.  With
 // 128-key tiles a wave holds two 128-key score tiles in flight and needs more
-// than the 256 VGPRs of two waves per SIMD, so the workgroup stays at 4 waves.
+// than the 256 VGPRs of two waves per SIMD, so the workgroup stays at 4 waves
+// (no rule takes them any more: fa_fwd; the exact entries and fa_supported do).
 // Counters (profiles/tile_study_mha_gqa_bwd.md, GQA B=2 H=32 H_kv=8 S=8192 D=128):
 // one head of 64 rows 898 TFLOP/s, MFMA busy 48.2 %; two heads 1185 / 71.4 %; four
 // heads 1236 / 68.4 %.

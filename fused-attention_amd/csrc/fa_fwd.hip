@@ -143,9 +143,11 @@ void fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K,
   const int wg = blockIdx.x;
   int unit, qt;
   if constexpr (KS > 1) {
-    // heaviest first over all heads (with a multiple of 8 heads an XCD still serves its own);
+    // heaviest first over all heads (with a multiple of 8 heads, those of one residue to an XCD);
     // when every workgroup is resident at once, the second one of a CU (from `first` on) in
-    // reverse, the lightest beside the heaviest (+1 to +4 % at B=2 H=8 S=2048, B=1 H=8 S=4096)
+    // reverse, the lightest beside the heaviest (+1 to +4 % at B=2 H=8 S=2048, B=1 H=8 S=4096).  The
+    // reversed half hands the heads of residue 7 - x to XCD x: each head's keys then pass through two
+    // L2s, which these figures include.
     const int L = first > 0 && wg >= first ? first + (int)gridDim.x - 1 - wg : wg;
     unit = L % nunits;
     qt = nq - 1 - L / nunits;
