@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <iterator>
 #include <mutex>
 
 #include "fa_launch.h"
@@ -167,13 +168,15 @@ bool short_rows(int B, int H, int S, int D) {
 //   B=2 H=8 S=2048 (512) 31.2 / 28.1 / 28.0 / 43.7; B=1 H=8 S=4096 (512) 56.2 / 49.7 / 44.3 / 68.0;
 //   GQA B=1 H=32 H_kv=8 S=1531 (768) 30.1 / 27.9 / 36.0 / 55.6; B=2 H=16 S=2048 (1024) 41.9 / 44.1 / 54 / 88
 // and the lengths from which the split pays, us of unsplit / split (heads of all batches, W; graph
-// replays, without the launches; at about 4000 sizes, groups of 1 to 32, the split calls now lie between
+// replays, without the launches; at about 4000 sizes, groups of 1 to 32, the split calls lie between
 // 0.29 and 1.03 of the unsplit ones, mean 0.81):
 //   W <= half the CUs: D = 64 S=64, 128 heads 4.20 / 4.41, S=100, 64 heads 5.21 / 4.46
 //   W <= one per CU: D = 64 S=64, 256 heads 4.39 / 5.33, GQA S=100, 128 heads 4.96 / 5.33, S=256, 64 heads 0.82 of it;
 //   D = 128: S=64, 128 heads 5.27 / 7.07, S=128, 128 heads 6.89 / 7.59, S=320 1.07, S=384, 42 heads 10.47 / 10.29
-//   W <= two: D = 64 S=512, 64 heads 9.66 / 7.56, MQA 19 / 12; D = 128 S=640, 48 heads 14.7 / 12.8, 51 heads
-//   15.9 / 16.6, S=1024, 25 heads 19.8 / 17.6
+//   W <= two: D = 64 S=512, 64 heads 9.66 / 7.56; D = 128 S=640, 48 heads 14.7 / 12.8, 51 heads 15.9 / 16.6,
+//   S=1024, 31 heads 20.3 / 20.9, S=1100, 25 heads 0.88
+//   W <= two and a quarter: D = 64 S=577, 56 heads 0.82 of it, GQA S=513, 62 heads 1.03; D = 128 S=640, 56 heads 0.87, S=576,
+//   60 heads 0.95, S=833, 41 heads 1.13
 //   W <= two and a half: D = 64 S=640, GQA, 64 heads 10.1 / 10.9, S=896, 45 heads 15.0 / 13.7; D = 128 S=833, 45
 //   heads 20.9 / 24.2, S=1280, 32 heads 26.6 / 22.9, 31 heads 26.2 / 28.1
 //   W <= three: GQA D = 64 S=640, 76 heads 10.6 / 12.5, S=1024, 48 heads 18.6 / 14.7, 44 heads 14.7 / 15.1, S=1531, 31
@@ -181,16 +184,25 @@ bool short_rows(int B, int H, int S, int D) {
 struct FwdShape {
   int block_m, block_n, gh;   // gh = -KS: key groups
 };
+constexpr int kNever = 0x7fffffff;
+struct KeySplitBand {
+  int quarters;             // up to this many quarters of a 64-row workgroup per CU
+  int narrow[2], wide[4];   // the longest S not split: D <= 64, heads any / a multiple of 8;
+                            // D = 128, heads odd / even / a multiple of 4 / of 8
+};
+constexpr KeySplitBand kKeySplit[] = {
+    {2, {64, 64}, {320, 320, 320, 320}},      {4, {128, 128}, {320, 320, 320, 320}},
+    {6, {511, 511}, {704, 511, 511, 511}},    {8, {511, 511}, {1024, 768, 511, 511}},
+    {9, {576, 576}, {1400, 768, 640, 640}},   {10, {832, 768}, {1400, 832, 832, 768}},
+    {12, {1280, 832}, {kNever, 1280, 1280, 832}},
+};
 bool fwd_key_split(int B, int H, int S, int D, FwdShape* out) {
   const long long heads = (long long)B * H, w = heads * ((S + 63) / 64), cus = cu_count();
-  int past;   // the longest S that is not split
-  if (2 * w <= cus) past = D == 128 ? 320 : 64;
-  else if (w <= cus) past = D == 128 ? 320 : 128;
-  else if (w <= 2 * cus) past = D < 128 || heads % 4 == 0 ? 511 : 896;
-  else if (2 * w <= 5 * cus) past = D < 128 || heads % 2 == 0 ? 832 : 1400;
-  else if (w <= 3 * cus && (D < 128 || heads % 2 == 0)) past = heads % 8 == 0 ? 832 : 1280;
-  else return false;
-  if (S <= past) return false;
+  const int pow2 = heads % 8 == 0 ? 3 : heads % 4 == 0 ? 2 : heads % 2 == 0 ? 1 : 0;
+  const KeySplitBand* band = kKeySplit;
+  while (4 * w > band->quarters * cus)
+    if (++band == std::end(kKeySplit)) return false;
+  if (S <= (D == 128 ? band->wide[pow2] : band->narrow[pow2 == 3])) return false;
   const bool four = w <= cus || (D == 128 && S >= 4096 && w <= 2 * cus);
   if (out) *out = !four ? FwdShape{64, 64, -2} : D == 128 ? FwdShape{64, 128, -4} : FwdShape{32, 128, -4};
   return true;

@@ -100,9 +100,11 @@ def test_nan_stays_in_its_row_block():
 # (heads, S, D, split): both sides of each band's shortest length
 ROUTES = [(4, 64, 32, False), (4, 65, 64, True), (4, 320, 128, False), (4, 321, 128, True),
           (128, 128, 64, False), (64, 129, 32, True), (64, 511, 64, False), (64, 512, 64, True),
-          (51, 640, 128, False), (48, 640, 128, True), (33, 897, 128, True), (64, 640, 32, False), (45, 896, 64, True),
-          (37, 1025, 128, False), (46, 1024, 128, False), (48, 1024, 128, True), (31, 1531, 128, False),
-          (36, 1281, 64, True), (48, 832, 64, False)]
+          (27, 704, 128, False), (27, 705, 128, True), (31, 1024, 128, False), (29, 1025, 128, True),
+          (42, 768, 128, False), (38, 769, 128, True), (48, 640, 128, True),
+          (64, 576, 32, False), (57, 577, 32, True), (60, 576, 128, False), (52, 641, 128, True), (41, 833, 128, False),
+          (64, 640, 32, False), (45, 832, 64, False), (45, 833, 64, True), (48, 769, 128, True), (37, 1025, 128, False),
+          (46, 1024, 128, False), (48, 1024, 128, True), (44, 1025, 64, False), (36, 1281, 64, True), (31, 1531, 128, False)]
 
 
 @pytest.mark.parametrize("H,S,D,split", ROUTES)
