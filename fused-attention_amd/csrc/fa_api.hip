@@ -274,30 +274,40 @@ int dkdv_nsplit(int B, int H, int H_kv, int S, int D) {
 }
 
 // Whether the backward runs as bwd_small_kernel: dQ and dK/dV in one launch of 64-row and 64-key
-// workgroups (a split dK/dV keeps its kernel behind that launch's dQ).  By the number W of 64-row
-// workgroups: at D = 128, whose workgroup has a CU to itself, up to one per CU; at D <= 64 up to two and
-// a half or three.  Less for short sequences: with one or two tiles to a chain there is
-// little to halve and the two launches are already short, so the twofold staging decides sooner.
-// Neither H_kv nor the workspace decides, so dQ is the same for all of them.
+// workgroups (a split dK/dV keeps its kernel behind that launch's dQ).  By the number W of dQ's 64-row
+// workgroups: at D = 128, whose workgroup has a CU to itself, up to one per CU; at D <= 64 up to three.
+// Within that the launch's dK/dV workgroups, W / group, bound it: the 128-key kernel has
+// half as many, so the fewer there are, the longer the one launch is ahead.  For MHA the bound is the
+// `quarters` of a workgroup per CU below: less for short sequences, where with one or two tiles to a
+// chain there is little to halve and the two launches are already short; a dK/dV workgroup weighs
+// five times a dQ one (fitted on groups of 1 to 8).  A split counts as MHA: there the launch is dQ alone.
+// The workspace does not decide, so dQ is the same with and without one.
 // Measured, us of the two kernels / the one launch (W):
 //   D = 32:  B=2 H=8 S=1024 (256) 27.6 / 15.5, B=1 H=16 S=2240 (560) 52.6 / 42.0, B=3 H=8 S=2048 (768) 68.0 /
-//   51.1, B=8 H=16 S=512 (1024) 24.3 / 25.5; 381 heads S=128 (762) 12.9 / 13.9, MQA 128 heads S=384 (768) 46.3 / 49.3
+//   51.1, B=8 H=16 S=512 (1024) 24.3 / 25.5; 381 heads S=128 (762) 12.9 / 13.9; groups of 2 to 8, W up to 768: 0.49 to
+//   0.99, mean 0.69; MQA 128 heads S=384 (768) 46.0 / 47.6
 //   D = 64:  B=2 H=8 S=512 (128) 23.4 / 12.2, B=2 H=16 S=1024 (512) 37.8 / 32.6, B=3 H=16 S=832 (624) 40.4 /
 //   34.7, B=4 H=16 S=1024 (1024) 54.9 / 58.3; 512 heads S=64 (512) 13.0 / 14.8, 251 heads S=128 (502) 15.4 /
 //   17.1, 384 heads S=128 (768) 20.5 / 23.5, 125 heads S=320 (625) 24.1 / 25.3, 75 heads S=600 (750) 35.3 / 38.0,
-//   16 heads S=3000 (752) 103 / 109
+//   24 heads S=2048 (768) 0.84, 16 heads S=3000 (752) 103 / 109; groups of 2 to 8: 0.49 to 1.02 (but of 2, 768 heads S=64
+//   17.8 / 19.0), mean 0.75; MQA 160 heads S=256 (640) 53.2 / 56.8
 //   D = 128: B=2 H=8 S=512 (128) 36.3 / 22.7, B=3 H=5 S=1000 (240) 56.5 / 46.3, B=2 H=8 S=1024 (256) 56.4 /
 //   45.2, B=3 H=8 S=768 (288) 47.2 / 47.8, B=4 H=16 S=512 (512) 39.9 / 59.0; 256 heads S=64 (256) 15.3 / 20.1, 128
-//   heads S=64 (128) 0.67 of the two kernels
+//   heads S=64 (128) 0.67; of groups 256 heads S=64: of 2 16.8 / 17.6, of 4 0.82
 //   dQ alone of a split: B=1 H=4 S=4096 D=128 137 / 124, D=64 94 / 87; B=2 H=8 H_kv=2 S=2048 D=64 73 / 70
-// At about 3900 sizes, groups of 1 to 32, the calls that take it lie between 0.44 and 1.03 of the
-// two kernels' time, mean 0.74.
-bool bwd_small(int B, int H, int S, int D) {
-  int quarters;   // of a 64-row workgroup per CU
+// At about 3700 sizes, groups of 1 to 32, the calls that take it lie between 0.44 and 1.04 of the
+// two kernels' time, mean 0.73.
+bool bwd_small(int B, int H, int H_kv, int S, int D) {
+  const long long tiles = (S + 63) / 64, dq = (long long)B * H * tiles, cus = cu_count();
+  if (dq > (D == 128 ? 1 : 3) * cus) return false;
+  const long long dkdv = dkdv_nsplit(B, H, H_kv, S, D) > 1 ? dq : (long long)B * H_kv * tiles;
+  int quarters;
   if (D == 128) quarters = S <= 64 ? 2 : 4;
-  else if (D == 64) quarters = S <= 48 ? 12 : S <= 64 ? 6 : S <= 128 ? 7 : S <= 384 ? 9 : S <= 640 ? 10 : 11;
-  else quarters = S <= 384 ? 10 : 12;
-  return 4LL * B * H * ((S + 63) / 64) <= (long long)quarters * cu_count();
+  else if (D == 32) quarters = S > 64 && S <= 384 ? 10 : 12;
+  else if (S <= 128) quarters = S <= 48 ? 12 : S <= 64 ? 6 : S <= 100 ? 10 : 7;
+  else if (S <= 640) quarters = S <= 384 ? 9 : 10;
+  else quarters = S <= 2048 && (long long)B * H % 8 == 0 ? 12 : 11;
+  return 2 * (dq + 5 * dkdv) <= 3 * quarters * cus;
 }
 
 // ---------------------------------------------------------------------------
@@ -371,7 +381,7 @@ int fa_bwd(const void* q, const void* k, const void* v, const void* o,
   fa::BwdFn fn = bwd_fn(dtype, D, B, H, S, block_m, block_n);
   if (!fn) return FA_ERR_UNSUPPORTED;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H, S, D, scale_log2, sm_scale, hip_stream,
-                nullptr, nullptr, 1, nullptr, false, bwd_small(B, H, S, D)};
+                nullptr, nullptr, 1, nullptr, false, bwd_small(B, H, H, S, D)};
   return fn(a);
 }
 
@@ -408,7 +418,7 @@ int fa_bwd_gqa(const void* q, const void* k, const void* v, const void* o,
   float* wsk = nsplit > 1 ? reinterpret_cast<float*>(ws) : nullptr;
   float* wsv = nsplit > 1 ? wsk + (size_t)B * H_kv * nsplit * S * D : nullptr;
   fa::BwdArgs a{q, k, v, o, d_o, lse, dq, dk, dv, B, H, H_kv, S, D, scale_log2, sm_scale, hip_stream,
-                wsk, wsv, nsplit, rowb, false, bwd_small(B, H, S, D)};
+                wsk, wsv, nsplit, rowb, false, bwd_small(B, H, H_kv, S, D)};
   return fn(a);
 }
 

@@ -53,22 +53,26 @@ def test_edges_of_the_rule(B, H, Hkv, S, D):
     check(q, k, v, do, (128, 64), f"small bwd edge B{B} H{H}/{Hkv} S{S} D{D}")
 
 
-# (heads, S, D, one launch): both sides of each bound
-ROUTES = [(128, 64, 128, True), (129, 64, 128, False), (128, 128, 128, True), (129, 100, 128, False),
-          (768, 48, 64, True), (769, 48, 64, False), (384, 64, 64, True), (385, 64, 64, False),
-          (224, 128, 64, True), (225, 128, 64, False), (144, 256, 64, True), (145, 256, 64, False),
-          (64, 640, 64, True), (65, 640, 64, False), (64, 704, 64, True), (65, 704, 64, False),
-          (106, 384, 32, True), (107, 384, 32, False), (109, 448, 32, True), (110, 448, 32, False)]
+# (heads, K/V heads, S, D, one launch): both sides of each bound
+ROUTES = [(128, 128, 64, 128, True), (129, 129, 64, 128, False), (128, 128, 128, 128, True), (129, 129, 100, 128, False),
+          (218, 109, 64, 128, True), (220, 110, 64, 128, False), (256, 64, 64, 128, True),
+          (768, 768, 48, 64, True), (769, 769, 48, 64, False), (384, 384, 64, 64, True), (385, 385, 64, 64, False),
+          (658, 329, 64, 64, True), (660, 330, 64, 64, False), (768, 192, 64, 64, True),
+          (320, 320, 100, 64, True), (321, 321, 100, 64, False), (224, 224, 128, 64, True), (225, 225, 128, 64, False),
+          (384, 192, 128, 64, True), (144, 144, 256, 64, True), (145, 145, 256, 64, False), (192, 96, 256, 64, True),
+          (64, 64, 640, 64, True), (65, 65, 640, 64, False), (65, 65, 704, 64, False), (64, 64, 768, 64, True),
+          (63, 63, 768, 64, False), (768, 768, 64, 32, True), (106, 106, 384, 32, True), (107, 107, 384, 32, False),
+          (128, 64, 384, 32, True), (109, 109, 448, 32, True), (110, 110, 448, 32, False)]
 
 
-@pytest.mark.parametrize("H,S,D,one", ROUTES)
-def test_where_the_backward_is_one_launch(H, S, D, one):
+@pytest.mark.parametrize("H,Hkv,S,D,one", ROUTES)
+def test_where_the_backward_is_one_launch(H, Hkv, S, D, one):
     """Calls that the one launch makes slower run the two kernels: bitwise the exact entry's, which always
     does.  A call of one launch differs from it by the fp32 summation order somewhere."""
     lib = _lib.load()
-    q, k, v, do = make(1, H, H, S, D, MANY_HEADS, seed=H + S)
+    q, k, v, do = make(1, H, Hkv, S, D, MANY_HEADS, seed=H + S)
     o, lse = _forward(q, k, v, 64, 64)
-    assert lib.fa_bwd_dkdv_split(1, H, H, S, D) == 1
+    assert lib.fa_bwd_dkdv_split(1, H, Hkv, S, D) == 1
     got = bwd(lib, q, k, v, o, do, lse, 64, 64)
     want = bwd(lib, q, k, v, o, do, lse, 64, 64, nsplit=1)
     assert all(torch.equal(a, b) for a, b in zip(got, want)) is not one
