@@ -94,6 +94,14 @@ using fa::kMaxDevices;
 // Interleaved timings, two heads of 128 rows against four of 64: GQA B=2 H=32 H_kv=8
 // S=8192 D=128 +0.8 %, B=1 H=32 H_kv=4 S=8192 +0.9 %, B=2 H=32 H_kv=8 S=4096 +1.5 %,
 // MQA B=1 H=32 S=16384 D=64 fp16 +0.3 %, B=2 H=32 H_kv=8 S=8192 D=64 fp16 +0.7 %.
+// The rows per head that the heads are chosen for: up to three 64-row workgroups per CU a
+// 128-row tile counts as 64, or a group's two heads of 128 rows would make half as many workgroups
+// of twice the chain (bitwise equal; us of 128 / 64 rows, two heads each, groups of 4: D = 128 128 heads S=100 8.7 /
+// 6.5, 128 heads S=256 12.9 / 9.8, 96 heads S=512 18.8 / 19.1; D = 64 256 heads S=64 4.9 / 4.6, 128 heads S=256 9.3 /
+// 6.7, 76 heads S=640 14.9 / 11.0; D = 32 48 heads S=1024 15.8 / 14.2).
+int fwd_tile_m(int B, int H, int S, int block_m) {
+  return (long long)B * H * ((S + 63) / 64) <= 3LL * cu_count() ? 64 : block_m;
+}
 int fwd_heads_per_wg(int B, int H, int group, int S, int D, int block_m, int block_n) {
   auto four_fit = [&](int bm) {
     return (long long)B * (H / 4) * ((S + bm - 1) / bm) >= (D <= 32 ? 4LL : 2LL) * cu_count();
@@ -361,9 +369,10 @@ int fa_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     // SIMD have, and is slower everywhere (us of 128 x 128 / 128 x 64, D = 32, 64, 128: MHA B=4
     // H=32 S=2048 89 / 62, 112 / 87, 189 / 139; GQA B=2 H=16 H_kv=4 S=4096 73 / 56, 97 / 77, 167 / 129;
     // B=16 H=32 S=512 D=32 47 / 29)
-    const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, 64);
+    const int tile_m = fwd_tile_m(B, H, S, block_m);
+    const int gh = fwd_heads_per_wg(B, H, H / H_kv, S, D, tile_m, 64);
     const bool few = gh == 1 && short_rows(B, H, S, D) && (long long)B * H * ((S + 63) / 64) > 2LL * cu_count();
-    w = FwdShape{few ? 64 : fwd_block_m(block_m, 64, D, gh), 64, gh};
+    w = FwdShape{few ? 64 : fwd_block_m(tile_m, 64, D, gh), 64, gh};
   }
   fa::FwdFn fn = fwd_table(dtype, D, w.block_m, w.block_n, w.gh, lse != nullptr);
   if (!fn) return FA_ERR_UNSUPPORTED;
@@ -493,7 +502,8 @@ int fa_fwd_heads_per_wg(int B, int H, int H_kv, int S, int D, int block_m, int b
   if (D != 32 && D != 64 && D != 128) return 0;
   if (!tile_ok(block_m) || !tile_ok(block_n)) return 0;
   if (fwd_key_split(B, H, S, D, nullptr)) return 1;
-  return fwd_heads_per_wg(B, H, H / H_kv, S, D, block_m, 64);   // (fa_fwd's tiles are 64 keys whatever block_n)
+  // (fa_fwd's tiles are 64 keys whatever block_n)
+  return fwd_heads_per_wg(B, H, H / H_kv, S, D, fwd_tile_m(B, H, S, block_m), 64);
 }
 
 int fa_fwd_rows_per_wg(int block_m, int block_n, int D, int heads_per_wg) {

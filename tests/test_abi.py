@@ -233,6 +233,8 @@ def test_exact_shape_entries_and_rule_queries(lib):
     assert lib.fa_fwd_heads_per_wg(1, 32, 1, 16384, 64, 128, 64) == 4
     assert lib.fa_fwd_heads_per_wg(2, 16, 4, 2048, 128, 128, 64) == 2   # four would leave CUs short
     assert lib.fa_fwd_heads_per_wg(2, 16, 4, 2048, 128, 64, 64) == 2  # 4 -> 2: under 2 workgroups per CU
+    assert lib.fa_fwd_heads_per_wg(3, 16, 2, 168, 128, 128, 64) == 2    # small grid, a 128-row tile as 64
+    assert lib.fa_fwd_heads_per_wg(64, 8, 2, 200, 64, 128, 64) == lib.fa_fwd_heads_per_wg(64, 8, 2, 200, 64, 64, 64) == 4
     assert lib.fa_fwd_heads_per_wg(2, 8, 1, 2048, 128, 128, 64) == 1    # one head, keys split over waves
     assert lib.fa_fwd_heads_per_wg(2, 8, 1, 1024, 128, 64, 64) == 1
     assert lib.fa_fwd_heads_per_wg(1, 16, 4, 4096, 128, 64, 64) == 2  # one per CU at four heads

@@ -141,6 +141,20 @@ def test_small_grids_run_the_shape_asked_for(B, H, Hkv, S, D, dtype):
         assert all(torch.equal(a, b[:B]) for a, b in zip(got, want)), f"backward, {bm} dQ rows"
 
 
+@pytest.mark.parametrize("B,H,Hkv,S,D,dtype", [
+    (2, 16, 4, 168, 128, torch.float16), (1, 128, 64, 65, 64, torch.bfloat16), (4, 64, 8, 150, 32, torch.float16),
+    (1, 250, 250, 130, 128, torch.bfloat16),
+])
+def test_forward_128_row_tile_of_a_small_grid_bitwise(B, H, Hkv, S, D, dtype):
+    """Up to three 64-row workgroups per CU (and not split over keys) a 128-row tile of grouped heads
+    counts as 64: the same O and LSE as two heads of 128 rows, and as tile 64."""
+    lib = _lib.load()
+    q, k, v, _ = inputs(B, H, Hkv, S, D, dtype, seed=S + H)
+    o, lse = fwd(lib, q, k, v, 128, 64)
+    for want in (fwd(lib, q, k, v, 64, 64), fwd(lib, q, k, v, 128, 64, min(2, H // Hkv))):
+        assert torch.equal(o, want[0]) and torch.equal(lse, want[1])
+
+
 @pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
 def test_forward_gqa_tile_as_four_heads_bitwise(D, dtype):
     """A 128-row, 64-key GQA tile runs as 64-row workgroups of four heads where the grid is large
