@@ -79,6 +79,15 @@ int check_common(int B, int H, int S, int D, int dtype, int block_m, int block_n
 using fa::cu_count;
 using fa::kMaxDevices;
 
+// The rows per head that the heads are chosen for: up to three 64-row workgroups per CU a
+// 128-row tile counts as 64, or a group's two heads of 128 rows would make half as many workgroups
+// of twice the chain (bitwise equal; us of 128 / 64 rows, two heads each, groups of 4: D = 128 128 heads S=100 8.7 /
+// 6.5, 128 heads S=256 12.9 / 9.8, 96 heads S=512 18.8 / 19.1; D = 64 256 heads S=64 4.9 / 4.6, 128 heads S=256 9.3 /
+// 6.7, 76 heads S=640 14.9 / 11.0; D = 32 48 heads S=1024 15.8 / 14.2).
+int fwd_tile_m(int B, int H, int S, int block_m) {
+  return (long long)B * H * ((S + 63) / 64) <= 3LL * cu_count() ? 64 : block_m;
+}
+
 // Forward query heads per workgroup for this launch: heads_per_wg's choice, but four
 // heads (64-row tiles) drop to two where the grid would leave the co-resident pair of
 // workgroups per CU short: below two workgroups per CU, and at D = 32 below four, where
@@ -94,14 +103,6 @@ using fa::kMaxDevices;
 // Interleaved timings, two heads of 128 rows against four of 64: GQA B=2 H=32 H_kv=8
 // S=8192 D=128 +0.8 %, B=1 H=32 H_kv=4 S=8192 +0.9 %, B=2 H=32 H_kv=8 S=4096 +1.5 %,
 // MQA B=1 H=32 S=16384 D=64 fp16 +0.3 %, B=2 H=32 H_kv=8 S=8192 D=64 fp16 +0.7 %.
-// The rows per head that the heads are chosen for: up to three 64-row workgroups per CU a
-// 128-row tile counts as 64, or a group's two heads of 128 rows would make half as many workgroups
-// of twice the chain (bitwise equal; us of 128 / 64 rows, two heads each, groups of 4: D = 128 128 heads S=100 8.7 /
-// 6.5, 128 heads S=256 12.9 / 9.8, 96 heads S=512 18.8 / 19.1; D = 64 256 heads S=64 4.9 / 4.6, 128 heads S=256 9.3 /
-// 6.7, 76 heads S=640 14.9 / 11.0; D = 32 48 heads S=1024 15.8 / 14.2).
-int fwd_tile_m(int B, int H, int S, int block_m) {
-  return (long long)B * H * ((S + 63) / 64) <= 3LL * cu_count() ? 64 : block_m;
-}
 int fwd_heads_per_wg(int B, int H, int group, int S, int D, int block_m, int block_n) {
   auto four_fit = [&](int bm) {
     return (long long)B * (H / 4) * ((S + bm - 1) / bm) >= (D <= 32 ? 4LL : 2LL) * cu_count();
@@ -183,8 +184,8 @@ bool short_rows(int B, int H, int S, int D) {
 //   D = 128: S=64, 128 heads 5.27 / 7.07, S=128, 128 heads 6.89 / 7.59, S=320 1.07, S=384, 42 heads 10.47 / 10.29
 //   W <= two: D = 64 S=512, 64 heads 9.66 / 7.56; D = 128 S=640, 48 heads 14.7 / 12.8, 51 heads 15.9 / 16.6,
 //   S=1024, 31 heads 20.3 / 20.9, S=1100, 25 heads 0.88
-//   W <= two and a quarter: D = 64 S=577, 56 heads 0.82 of it, GQA S=513, 62 heads 1.03; D = 128 S=640, 56 heads 0.87, S=576,
-//   60 heads 0.95, S=833, 41 heads 1.13
+//   W <= two and a quarter: D = 64 S=577, 56 heads 0.82 of it, GQA S=513, 62 heads 1.03; D = 128 S=640, 56
+//   heads 0.87, S=576, 60 heads 0.95, S=833, 41 heads 1.13
 //   W <= two and a half: D = 64 S=640, GQA, 64 heads 10.1 / 10.9, S=896, 45 heads 15.0 / 13.7; D = 128 S=833, 45
 //   heads 20.9 / 24.2, S=1280, 32 heads 26.6 / 22.9, 31 heads 26.2 / 28.1
 //   W <= three: GQA D = 64 S=640, 76 heads 10.6 / 12.5, S=1024, 48 heads 18.6 / 14.7, 44 heads 14.7 / 15.1, S=1531, 31
